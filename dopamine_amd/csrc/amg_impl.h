@@ -17,17 +17,20 @@
 //   aggregate: strongly anisotropic cells give line aggregates), the first aggregation is redone
 //   with a small threshold (every coupling strong: compact 3-D aggregates of about 9 cells) and
 //   the cycle uses the larger over-correction alpha = 2 (AmgCfg::theta0, min_ratio0, alpha_aggr);
-// - one application is a V(1,1) cycle: per level a damped-Jacobi pre-smoothing step from zero
-//   fused with the residual, a gather restriction over each aggregate's children, the dense solve
-//   at the bottom, and the prolongation (scaled by alpha, the over-correction that unsmoothed
-//   aggregation needs) fused with a damped-Jacobi post-smoothing step. Pre- and post-smoothing are
-//   the same operator, so the cycle is a fixed symmetric linear map;
+// - one application is a V(1,1) cycle with damped-Jacobi smoothing (pre-smoothing from zero, pre-
+//   and post-smoothing the same operator, so the cycle is a fixed symmetric linear map). Every
+//   coarse level is two sparse products: the way down applies the pre-smoothed restriction
+//   R = P^T (I - w A D^-1), the way up y = (2 w D^-1 - w^2 D^-1 A D^-1) b + alpha R^T y_coarse
+//   (alpha: the over-correction that unsmoothed aggregation needs), with R formed at set-up. No
+//   smoothed vector or residual is stored between them. The bottom is one dense product: the
+//   inverse of the coarsest operator, or, where the level above it is still small, that whole
+//   level's cycle as a matrix (AmgCfg::dense_max);
 // - everything is FP32 (operator values, vectors); the flexible CG around it keeps its dot
 //   products in FP64 and, in mixed precision, sits inside FP64 iterative refinement.
 //
 // Stored coefficients: cs_ij = coef_ij / diag_j (the pre-smoothing residual
-// r = b - A (w D^-1 b) = (1 - w) b + w sum_j cs_ij b_j needs no neighbour diagonals) and
-// cr_ij = coef_ij / diag_i (the post-smoothing step y = x + w (D^-1 b - x + sum_j cr_ij x_j)).
+// r = b - A (w D^-1 b) = (1 - w) b + w sum_j cs_ij b_j needs no neighbour diagonals) and, on level
+// 0, cr_ij = coef_ij / diag_i (its post-smoothing y = x + w (D^-1 b - x + sum_j cr_ij x_j)).
 #pragma once
 
 #include "cg_impl.h"
@@ -249,6 +252,95 @@ inline void amg_dense_inverse(const AmgOp& C, std::vector<float>& inv, bool* sin
   }
 }
 
+// The pre-smoothed restriction R = P^T (I - w A D^-1) as CSR (columns ascending within a row):
+// R_Ii = (1 - w) [i in I] + w sum of cs_ci over the children c of I. scaled(c, q, &cs) gives the
+// scaled coupling of entry q of row c, or false where it is left out of the smoothing.
+struct AmgCsr {
+  std::vector<int> ptr, col;
+  std::vector<double> val;
+};
+template <class Scaled>
+inline AmgCsr amg_restriction(const AmgOp& A, double omega, int na, const std::vector<int>& kptr,
+                              const std::vector<int>& kidx, Scaled&& scaled) {
+  AmgCsr R;
+  R.ptr.assign(size_t(na) + 1, 0);
+  std::vector<std::pair<int, double>> row;
+  for (int I = 0; I < na; ++I) {
+    row.clear();
+    for (int q = kptr[I]; q < kptr[I + 1]; ++q) {
+      const int c = kidx[q];
+      row.push_back({c, 1.0 - omega});
+      for (int k = 0; k < A.w; ++k) {
+        const size_t e = size_t(k) * A.n + c;
+        double cs;
+        if (scaled(c, e, &cs)) row.push_back({A.nbr[e], omega * cs});
+      }
+    }
+    std::sort(row.begin(), row.end());
+    for (size_t q = 0; q < row.size(); ++q) {
+      if (int(R.col.size()) > R.ptr[I] && R.col.back() == row[q].first) {
+        R.val.back() = R.val.back() + row[q].second;
+      } else {
+        R.col.push_back(row[q].first);
+        R.val.push_back(row[q].second);
+      }
+    }
+    R.ptr[size_t(I) + 1] = int(R.col.size());
+  }
+  return R;
+}
+inline AmgCsr amg_transpose(const AmgCsr& R, int n_cols) {
+  AmgCsr T;
+  const int n = int(R.ptr.size()) - 1;
+  T.ptr.assign(size_t(n_cols) + 1, 0);
+  for (int c : R.col) T.ptr[size_t(c) + 1]++;
+  for (int c = 0; c < n_cols; ++c) T.ptr[size_t(c) + 1] += T.ptr[c];
+  T.col.assign(R.col.size(), 0);
+  T.val.assign(R.col.size(), 0.0);
+  std::vector<int> at(T.ptr.begin(), T.ptr.end() - 1);
+  for (int I = 0; I < n; ++I)
+    for (int q = R.ptr[I]; q < R.ptr[I + 1]; ++q) {
+      const int p = at[R.col[q]]++;
+      T.col[p] = I;
+      T.val[p] = R.val[q];
+    }
+  return T;
+}
+
+// A level's cycle as a matrix, given the one of the level below (M, nb x nb): T + alpha R^T M R
+// with T = 2 w D^-1 - w^2 D^-1 A D^-1.
+template <class Scaled>
+inline std::vector<float> amg_fold(const AmgOp& A, const AmgCsr& R, const std::vector<float>& M, double omega,
+                                   double alpha, const std::vector<float>& dinv, Scaled&& scaled) {
+  const int n = A.n, nb = int(R.ptr.size()) - 1;
+  std::vector<double> X(size_t(nb) * n, 0.0);  // M R
+  for (int I = 0; I < nb; ++I)
+    for (int q = R.ptr[I]; q < R.ptr[I + 1]; ++q) {
+      const int j = R.col[q];
+      for (int K = 0; K < nb; ++K) X[size_t(K) * n + j] += double(M[size_t(K) * nb + I]) * R.val[q];
+    }
+  std::vector<double> row(n);
+  std::vector<float> out(size_t(n) * n);
+  const AmgCsr Q = amg_transpose(R, n);
+  for (int c = 0; c < n; ++c) {
+    std::fill(row.begin(), row.end(), 0.0);
+    for (int q = Q.ptr[c]; q < Q.ptr[c + 1]; ++q) {
+      const double f = alpha * Q.val[q];
+      const double* x = &X[size_t(Q.col[q]) * n];
+      for (int j = 0; j < n; ++j) row[j] += f * x[j];
+    }
+    const double di = omega * double(dinv[c]);
+    row[c] += di * (2.0 - omega);
+    for (int k = 0; k < A.w; ++k) {
+      const size_t e = size_t(k) * n + c;
+      double cs;
+      if (scaled(c, e, &cs)) row[A.nbr[e]] += di * omega * cs;
+    }
+    for (int j = 0; j < n; ++j) out[size_t(c) * n + j] = float(row[j]);
+  }
+  return out;
+}
+
 struct AmgCfg {
   double theta = 0.08;       // strength threshold
   double omega = 0.8;        // Jacobi damping
@@ -262,6 +354,10 @@ struct AmgCfg {
   double min_ratio0 = 3.5;
   double alpha_aggr = 2.4;
   int coarse_max = 1500;     // cells of the densely solved level
+  // Levels of at most dense_max cells above it are folded into it: their cycle as one dense
+  // product instead of three kernels (2,457 cells on the channel: 24 MB in 5.9 us, where the
+  // three took 3 x 3-4 us; the line lies where the matrix takes as long to read as the kernels).
+  int dense_max = 2816;
   int max_levels = 16;
 };
 
@@ -269,29 +365,13 @@ struct AmgCfg {
 
 // One level in the execution space. Level 0 keeps the operator's ELL lists (one thread per cell,
 // the solver's own neighbour array).
-// Coarse levels store their rows, and every level the children lists of the next coarser level's
-// cells, as sliced ELL: slices of AMG_SL rows (one wavefront), each as wide as its longest row,
-// entry k of row r at sptr[r / AMG_SL] + k AMG_SL + r % AMG_SL. One lane per row then reads a
-// contiguous 256-byte line per slot with no reduction across lanes. Row padding points at the row
-// itself with zero coefficients; children padding is -1.
-constexpr int AMG_SL = 64;
-constexpr int AMG_UN = 4;  // slice widths are multiples of this: each lane keeps 4 independent loads in flight
-
-// Slot of every CSR entry in the sliced-ELL layout; sptr gets the slice offsets. Returns the size.
-inline size_t amg_sell_layout(int n, const std::vector<int>& rptr, std::vector<int>& sptr, std::vector<int>& pos) {
-  const int nsl = (n + AMG_SL - 1) / AMG_SL;
-  sptr.assign(size_t(nsl) + 1, 0);
-  for (int sl = 0; sl < nsl; ++sl) {
-    int w = 0;
-    for (int r = sl * AMG_SL; r < std::min(n, (sl + 1) * AMG_SL); ++r) w = std::max(w, rptr[r + 1] - rptr[r]);
-    w = (w + AMG_UN - 1) / AMG_UN * AMG_UN;
-    sptr[size_t(sl) + 1] = sptr[sl] + w * AMG_SL;
-  }
-  pos.assign(size_t(rptr[n]), 0);
-  for (int r = 0; r < n; ++r)
-    for (int q = rptr[r]; q < rptr[r + 1]; ++q) pos[q] = sptr[r / AMG_SL] + (q - rptr[r]) * AMG_SL + r % AMG_SL;
-  return size_t(sptr[nsl]);
-}
+// The sparse matrices of the cycle are packed rows: row r's entries from 4 ptr[r] to 4 ptr[r + 1],
+// padded to groups of AMG_UN entries (the row's first column again, with zero values). Several
+// lanes take a row, a lane reads a group's columns and values in one 16-byte load each, and
+// neighbouring lanes and rows read neighbouring memory. In sliced ELL with the same lanes per row
+// a row's entries lie 256 bytes apart: the products on the channel's levels of 198,654 and 53,495
+// rows took 10.2 us, packed 6.7 us (mean of the three upward ones).
+constexpr int AMG_UN = 4;
 
 // The smoothers' scaled couplings cs = coef / diag_j, cr = coef / diag_i lie in [0, 1] and are
 // stored as IEEE binary16 (AmgCoef): half the bytes of the smoothing passes' coefficient stream.
@@ -346,23 +426,30 @@ inline AmgCoef coef_h(float f) {
   return AmgCoef(sign | r);
 }
 
+// A sparse matrix in packed rows, with FP32 or binary16 values.
+template <class V>
+struct AmgMat {
+  const int *ptr = nullptr, *col = nullptr;
+  const V* val = nullptr;
+};
+
 struct AmgLevelDev {
   int n = 0, w = 0;                              // cells; ELL width (level 0 only)
   const int* nbr = nullptr;                      // level 0: ELL neighbours [slot][cell]
-  const int *sptr = nullptr, *col = nullptr;     // coarse levels: sliced-ELL rows
-  const AmgCoef *cs = nullptr, *cr = nullptr;
+  const AmgCoef *cs = nullptr, *cr = nullptr;    // level 0: scaled couplings [slot][cell]
   // level 0, when its neighbour offsets fit 16 bits (EllOff16): each slot's coupling and offset
   // in one word (binary16 coupling in the low half, offset - obase[slot] in the high half)
   const uint32_t *hs = nullptr, *hr = nullptr;
   int obase[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   const float* dinv = nullptr;
-  const int *kptr = nullptr, *kidx = nullptr;    // children (cells of this level) of the next coarser level's cells, sliced ELL
-  float *b = nullptr, *x = nullptr, *r = nullptr;
-  // level 0 with three or more levels: its cells' aggregates and level 1's post-smoothed values,
-  // prolongated by a streaming pass (Prolong0)
+  AmgMat<AmgCoef> S;                             // coarse levels: the couplings cs
+  AmgMat<float> R, Q;                            // R to the next level; coarse levels: Q = R^T
+  float *b = nullptr, *y = nullptr;              // coarse levels: right-hand side, correction
+  float* x = nullptr;                            // level 0: what the post-smoothing starts from
+  // level 0: its cells' aggregates and level 1's correction, prolongated by a streaming pass
+  // (Prolong0)
   const int* agg = nullptr;
   const float* yc = nullptr;
-  float* y = nullptr;  // level 1: the post-smoothed values the finest level reads
 };
 
 namespace amgk {
@@ -373,9 +460,18 @@ namespace amgk {
 // (sets inner_done).
 enum Mode { OUTER = 0, INNER = 1 };
 
-DM_INLINE bool gated(const CgScalars* sc, int mode) { return sc && (sc->done || (mode == INNER && sc->inner_done)); }
+// Both flags are read before either is tested, so the two loads travel together with whatever
+// else the kernel has issued. Level 0's kernels test it first (a pass after convergence returns at
+// once); the coarse levels' kernels, where a dependent load costs more than the work, compute
+// first and let it decide the stores.
+DM_INLINE bool gated(const CgScalars* sc, int mode) {
+  if (!sc) return false;
+  const int d = sc->done, e = sc->inner_done;
+  return (d | (mode == INNER ? e : 0)) != 0;
+}
 
 DM_INLINE bool cycle_test(CgScalars* sc, int mode, int k, double rr, bool leader) {
+  if (!sc) return true;  // a cycle outside a solve
   if (gated(sc, mode)) return false;
   if (mode == OUTER) {
     const int fin = (sqrt(rr) <= sc->ttol) ? 1 : (k >= sc->maxit ? 2 : 0);
@@ -422,23 +518,6 @@ DM_INLINE bool group_lane(int t, int* lane, int* stride) {
 #endif
 }
 
-// pre-smoothing from zero and its residual, level 0 (ELL): x = w D^-1 b,
-// r = (1 - w) b + w sum_j cs_ij b_j
-template <class T>
-DM_INLINE void down_cell(const AmgLevelDev& L, const T* b, float omega, int c) {
-  const int n = L.n;
-  const float bc = float(b[c]);
-  float s = 0.0f;
-  for (int k = 0; k < L.w; ++k) {
-    const size_t q = size_t(k) * n + c;
-    const int j = L.nbr[q];
-    if (j < 0) continue;
-    s = s + coef_f(L.cs[q]) * float(b[j]);
-  }
-  L.x[c] = omega * L.dinv[c] * bc;
-  L.r[c] = (1.0f - omega) * bc + omega * s;
-}
-
 // post-smoothing, level 0 (ELL), x already holding the prolongated coarse correction:
 // y = x + w (D^-1 b - x + sum_j cr_ij x_j)
 template <class T>
@@ -456,17 +535,20 @@ DM_INLINE float up_cell(const AmgLevelDev& L, const T* b, float omega, float al,
   return xc + omega * (L.dinv[c] * float(b[c]) - xc + s);
 }
 
-// the prolongation of level 1's post-smoothed values into level 0 as a streaming pass over the
-// fine cells: x += alpha y_c[agg] (coalesced reads of x and agg, y_c resident in L2), instead of
-// each coarse cell scattering into its children
+// The vector that level 0's post-smoothing starts from, as a streaming pass over the fine cells:
+// the pre-smoothed b (formed again here rather than stored by the way down) plus the prolongated
+// correction, x = w D^-1 b + alpha y_c[agg] (coalesced reads of b, D^-1 and agg, y_c resident in
+// L2).
+template <class T>
 struct Prolong0 {
   AmgLevelDev L;
+  const T* b;
   const CgScalars* sc;
   int mode;
-  float al;
+  float omega, al;
   DM_HD void operator()(int c) const {
     if (gated(sc, mode)) return;
-    L.x[c] = L.x[c] + al * L.yc[L.agg[c]];
+    L.x[c] = omega * L.dinv[c] * float(b[c]) + al * L.yc[L.agg[c]];
   }
 };
 
@@ -496,52 +578,7 @@ DM_INLINE void slots0p(const AmgLevelDev& L, const uint32_t* hw, int c, int* jj,
   }
 }
 
-// level 0 pre-smoothing as a chained pass: its setup is the convergence test of iteration k
-template <class T, int WC = 0>
-struct Down0 {
-  static constexpr int kSlots = WC;
-  AmgLevelDev L;
-  const T* b;
-  CgScalars* sc;
-  int mode, k;
-  float omega;
-  using Scal = cgk::NoScal;
-  DM_HD bool setup(const Red<1>& t, bool leader, Scal&) const { return cycle_test(sc, mode, k, t.v[0], leader); }
-  DM_HD Red<1> operator()(int c, const Scal&) const {
-    down_cell(L, b, omega, c);
-    Red<1> o;
-    o.v[0] = 0.0;
-    return o;
-  }
-  DM_HD Red<1> run(int lo, int hi, int t, int nt, const Scal&) const {
-    for (int c = lo + t; c < hi; c += nt) {
-      int jj[WC > 0 ? WC : 1];
-      float h[WC > 0 ? WC : 1], bj[WC > 0 ? WC : 1];
-      if (L.hs)
-        slots0p<WC>(L, L.hs, c, jj, h);
-      else
-        slots0<WC>(L, L.cs, c, jj, h);
-#pragma unroll
-      for (int kk = 0; kk < WC; ++kk) bj[kk] = float(b[jj[kk]]);
-      const float bc = float(b[c]);
-      float s = 0.0f;
-#pragma unroll
-      for (int kk = 0; kk < WC; ++kk) s = s + h[kk] * bj[kk];
-      L.x[c] = omega * L.dinv[c] * bc;
-      L.r[c] = (1.0f - omega) * bc + omega * s;
-    }
-    return red_identity<1, false>();
-  }
-};
-
-// the same level-0 steps outside a solve (one V-cycle on its own)
-template <class T>
-struct Down0F {
-  AmgLevelDev L;
-  const T* b;
-  float omega;
-  DM_HD void operator()(int c) const { down_cell(L, b, omega, c); }
-};
+// the level-0 post-smoothing outside a solve (one V-cycle on its own)
 template <class T>
 struct Up0F {
   AmgLevelDev L;
@@ -551,154 +588,165 @@ struct Up0F {
   DM_HD void operator()(int c) const { z[c] = T(up_cell(L, r, omega, al, c)); }
 };
 
-// Row slot helpers of the sliced-ELL layout: the first slot of row r and the slice's width.
-DM_INLINE int sell_base(const int* sptr, int r) { return sptr[r / AMG_SL] + r % AMG_SL; }
-DM_INLINE int sell_width(const int* sptr, int r) { return (sptr[r / AMG_SL + 1] - sptr[r / AMG_SL]) / AMG_SL; }
-// sum_k a_rk v[col_rk] over this lane's chunks of AMG_UN slots of row r (chunks lane, lane + st,
-// ...), AMG_UN independent loads at a time
-DM_INLINE float sell_row(const int* sptr, const int* col, const AmgCoef* a, const float* v, int r, int lane, int st) {
-  const int q0 = sell_base(sptr, r), nch = sell_width(sptr, r) / AMG_UN;
-  float s = 0.0f;
-  for (int ch = lane; ch < nch; ch += st) {
-    const int k = ch * AMG_UN;
-    int j[AMG_UN];
-    float h[AMG_UN], x[AMG_UN];
-#pragma unroll
-    for (int u = 0; u < AMG_UN; ++u) {
-      j[u] = col[q0 + (k + u) * AMG_SL];
-      h[u] = coef_f(a[q0 + (k + u) * AMG_SL]);
-    }
-#pragma unroll
-    for (int u = 0; u < AMG_UN; ++u) x[u] = v[j[u]];
-#pragma unroll
-    for (int u = 0; u < AMG_UN; ++u) s = s + h[u] * x[u];
-  }
-  return s;
+// Lanes per row: about one per group of four entries (rows of S and Q hold 8 to 16 entries, rows of
+// R 20 to 40).
+constexpr int AMG_GR = 8, AMG_GU = 4;
+
+struct alignas(16) AmgI4 {
+  int v[4];
+};
+struct alignas(16) AmgF4 {
+  float v[4];
+};
+struct alignas(8) AmgH4 {
+  AmgCoef v[4];
+};
+DM_INLINE AmgF4 group4(const float* p) { return *reinterpret_cast<const AmgF4*>(p); }
+DM_INLINE AmgF4 group4(const AmgCoef* p) {
+  const AmgH4 h = *reinterpret_cast<const AmgH4*>(p);
+  return AmgF4{{coef_f(h.v[0]), coef_f(h.v[1]), coef_f(h.v[2]), coef_f(h.v[3])}};
 }
 
-// Lanes per row: one on the large levels (every wavefront reads whole 256-byte slot lines), four
-// on levels of fewer rows, where the serial slot loop would leave the level latency-bound.
-constexpr int AMG_SMALL_ROWS = 1 << 18;
+// One group of AMG_UN entries of a row: its columns and values first, then what it gathers, so
+// that groups of different matrices travel together. A group past the row's end reads the row's
+// first one with zero values.
+struct RowGroup {
+  AmgI4 j;
+  AmgF4 h;
+  template <class V>
+  DM_INLINE void load(const AmgMat<V>& m, int q0, int g, int ng) {
+    const bool live = g < ng;
+    const int q = (q0 + (live ? g : 0)) * AMG_UN;
+    j = *reinterpret_cast<const AmgI4*>(m.col + q);
+    h = group4(m.val + q);
+#pragma unroll
+    for (int u = 0; u < AMG_UN; ++u) h.v[u] = live ? h.v[u] : 0.0f;
+  }
+  template <class T>
+  DM_INLINE float dot(const T* x) const {
+    float v[AMG_UN], s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < AMG_UN; ++u) v[u] = float(x[j.v[u]]);
+#pragma unroll
+    for (int u = 0; u < AMG_UN; ++u) s = s + h.v[u] * v[u];
+    return s;
+  }
+};
+// (R x)_r by the G lanes of a group
+template <int G, class T>
+DM_INLINE float row_dot(const AmgMat<float>& m, const T* x, int r, int lane, int st) {
+  const int q0 = m.ptr[r], ng = m.ptr[r + 1] - q0;
+  float s = 0.0f;
+  for (int g = lane; g < ng; g += st) {
+    RowGroup c;
+    c.load(m, q0, g, ng);
+    s = s + c.dot(x);
+  }
+  return group_sum<G>(s);
+}
 
-// b_coarse[I] = sum of the fine residual over aggregate I's cells (G lanes per aggregate)
-template <int G>
-struct Restrict {
-  const int *kptr, *kidx;
-  const float* rf;
-  float* bc;
+// A coarse level on the way down: the next level's right-hand side b_next = R b.
+struct RestrictS {
+  AmgMat<float> R;
+  const float* b;
+  float* bn;
   const CgScalars* sc;
   int mode;
   DM_HD void operator()(int t) const {
     int lane, st;
-    if (!group_lane<G>(t, &lane, &st)) return;
-    if (gated(sc, mode)) return;
-    const int I = t / G;
-    const int q0 = sell_base(kptr, I), nch = sell_width(kptr, I) / AMG_UN;
-    float s = 0.0f;
-    for (int ch = lane; ch < nch; ch += st) {
-      const int k = ch * AMG_UN;
-      int i[AMG_UN];
-      float v[AMG_UN];
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u) i[u] = kidx[q0 + (k + u) * AMG_SL];
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u) v[u] = i[u] >= 0 ? rf[i[u]] : 0.0f;
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u) s = s + v[u];
-    }
-    s = group_sum<G>(s);
-    if (lane == 0) bc[I] = s;
+    if (!group_lane<AMG_GR>(t, &lane, &st)) return;
+    const bool off = gated(sc, mode);
+    const float s = row_dot<AMG_GR>(R, b, t / AMG_GR, lane, st);
+    if (lane == 0 && !off) bn[t / AMG_GR] = s;
   }
 };
 
-// coarse-level pre-smoothing and residual (G lanes per row)
-template <int G>
-struct DownC {
-  AmgLevelDev L;
-  const CgScalars* sc;
-  int mode;
-  float omega;
-  DM_HD void operator()(int t) const {
-    int lane, st;
-    if (!group_lane<G>(t, &lane, &st)) return;
-    if (gated(sc, mode)) return;
-    const int c = t / G;
-    const float s = group_sum<G>(sell_row(L.sptr, L.col, L.cs, L.b, c, lane, st));
-    if (lane == 0) {
-      const float bc = L.b[c];
-      L.x[c] = omega * L.dinv[c] * bc;
-      L.r[c] = (1.0f - omega) * bc + omega * s;
+// The same from level 0 as a chained pass whose setup is the convergence test of iteration k. Reads
+// R (256 B per aggregate of 9 cells) and gathers b in place of the smoothing pass over the cells and
+// the gather of its residual over the aggregates: 8.8 us for 13.0 us on 509,486 cells, 11.9 us for
+// 17.6 us on 786,432; at 7.9 million (HBM-bound) 93 us for 92 us.
+template <class T>
+struct Restrict0 {
+  static constexpr int kSlots = 1;
+  AmgMat<float> R;
+  const T* b;
+  float* bn;
+  CgScalars* sc;
+  int mode, k;
+  using Scal = cgk::NoScal;
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal&) const { return cycle_test(sc, mode, k, t.v[0], leader); }
+  DM_HD Red<0> run(int lo, int hi, int t, int nt, const Scal&) const {
+    for (int q = lo + t; q < hi; q += nt) {
+      int lane, st;
+      if (!group_lane<AMG_GR>(q, &lane, &st)) continue;
+      const float s = row_dot<AMG_GR>(R, b, q / AMG_GR, lane, st);
+      if (lane == 0) bn[q / AMG_GR] = s;
     }
+    return Red<0>{};
   }
 };
 
-// Coarse-level post-smoothing (G lanes per row), then the prolongation with over-correction into
-// the next finer level: x_fine[i] += alpha y for the cell's children i (each fine cell has one
-// parent, so the writes never collide).
-template <int G>
-struct UpC {
+// A coarse level on the way up: y = w D^-1 ((2 - w) b + w sum_j cs_j b_j) + alpha Q y_next, the
+// pre-smoothing, the coarse correction and the post-smoothing in one.
+struct UpS {
   AmgLevelDev L;
-  const int *kptr, *kidx;  // this level's cells' children on the finer level
-  float* xf;
+  const float* yn;
   const CgScalars* sc;
   int mode;
   float omega, alpha;
-  float* yout = nullptr;  // level 1 under a level 0 that prolongates itself: store y, no scatter
   DM_HD void operator()(int t) const {
     int lane, st;
-    if (!group_lane<G>(t, &lane, &st)) return;
-    if (gated(sc, mode)) return;
-    const int c = t / G;
-    const float s = group_sum<G>(sell_row(L.sptr, L.col, L.cr, L.x, c, lane, st));
-    const float xc = L.x[c];
-    const float y = xc + omega * (L.dinv[c] * L.b[c] - xc + s);
-    if (yout) {
-      if (lane == 0) yout[c] = y;
-      return;
+    if (!group_lane<AMG_GU>(t, &lane, &st)) return;
+    const bool off = gated(sc, mode);
+    const int c = t / AMG_GU;
+    const int q0 = L.S.ptr[c], nq = L.S.ptr[c + 1] - q0, p0 = L.Q.ptr[c], np = L.Q.ptr[c + 1] - p0;
+    const float bc = L.b[c], di = omega * L.dinv[c];
+    float s = 0.0f, p = 0.0f;
+    for (int g = lane; g < nq || g < np; g += st) {
+      RowGroup a, q;  // a cell has at least its own aggregate in Q; its row of S may be empty
+      if (nq > 0) a.load(L.S, q0, g, nq);
+      q.load(L.Q, p0, g, np);
+      if (nq > 0) s = s + a.dot(L.b);
+      p = p + q.dot(yn);
     }
-    const float a = alpha * y;
-    const int p0 = sell_base(kptr, c), nch = sell_width(kptr, c) / AMG_UN;
-    for (int ch = lane; ch < nch; ch += st) {
-      const int k = ch * AMG_UN;
-      int i[AMG_UN];
-      float v[AMG_UN];
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u) i[u] = kidx[p0 + (k + u) * AMG_SL];
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u) v[u] = i[u] >= 0 ? xf[i[u]] : 0.0f;
-#pragma unroll
-      for (int u = 0; u < AMG_UN; ++u)
-        if (i[u] >= 0) xf[i[u]] = v[u] + a;
-    }
+    const float v = group_sum<AMG_GU>(di * (omega * s) + alpha * p);
+    if (lane == 0 && !off) L.y[c] = v + di * ((2.0f - omega) * bc);
   }
 };
 
-// Coarsest level: y = inv b (dense, symmetric, a wavefront per row), then the prolongation into
-// the next finer level as in UpC.
+// The bottom of the cycle: y = M b, M dense and row-major with rows padded to lda (a multiple of
+// 4, zeros), a wavefront per row, four 16-byte loads in flight per lane.
 constexpr int AMG_GC = 64;
-struct Coarsest {
-  int n;
-  const float* inv;
-  const float* b;
-  const int *kptr, *kidx;
-  float* xf;
+struct DenseS {
+  int lda;
+  const float *M, *b;
+  float* y;
   const CgScalars* sc;
   int mode;
-  float alpha;
   DM_HD void operator()(int t) const {
     int lane, st;
     if (!group_lane<AMG_GC>(t, &lane, &st)) return;
-    if (gated(sc, mode)) return;
-    const int i = t / AMG_GC;
+    const bool off = gated(sc, mode);
+    const int i = t / AMG_GC, nq = lda / 4;
+    const AmgF4* m4 = reinterpret_cast<const AmgF4*>(M + size_t(i) * lda);
+    const AmgF4* b4 = reinterpret_cast<const AmgF4*>(b);
     float s = 0.0f;
-    for (int j = lane; j < n; j += st) s = s + inv[size_t(i) * n + j] * b[j];
-    s = group_sum<AMG_GC>(s);
-    const float a = alpha * s;
-    const int p0 = sell_base(kptr, i), pw = sell_width(kptr, i);
-    for (int k = lane; k < pw; k += st) {
-      const int c = kidx[p0 + k * AMG_SL];
-      if (c >= 0) xf[c] = xf[c] + a;
+    for (int k0 = lane; k0 < nq; k0 += 4 * st) {
+      AmgF4 m[4], v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + u * st < nq ? k0 + u * st : k0;
+        m[u] = m4[k];
+        v[u] = b4[k];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float d = (m[u].v[0] * v[u].v[0] + m[u].v[1] * v[u].v[1]) + (m[u].v[2] * v[u].v[2] + m[u].v[3] * v[u].v[3]);
+        s = s + (k0 + u * st < nq ? d : 0.0f);
+      }
     }
+    s = group_sum<AMG_GC>(s);
+    if (lane == 0 && !off) y[i] = s;
   }
 };
 
@@ -716,7 +764,7 @@ struct Up0 {
   int mode;
   float omega, al;
   using Scal = cgk::NoScal;
-  DM_HD bool setup(const Red<1>&, bool, Scal&) const { return !gated(sc, mode); }
+  DM_HD bool setup(const Red<0>&, bool, Scal&) const { return !gated(sc, mode); }
   DM_HD Red<5> operator()(int c, const Scal&) const {
     const float y = up_cell(L, r, omega, al, c);
     const T zc = T(y);
@@ -773,101 +821,63 @@ class AmgPc : public FcgPc, public FcgPc32 {
     cfg_ = cfg;
     alpha_ = cfg.alpha;
     aggressive_ = false;
-    const int* agg0 = nullptr;
-    AmgOp cur = A;
-    for (int lev = 0;; ++lev) {
-      AmgLevelDev L;
-      L.n = cur.n;
-      // cs_ij = coef_ij / diag_j, cr_ij = coef_ij / diag_i, dinv_i = 1 / diag_i; a cell whose
-      // diagonal vanishes (an aggregate that is a whole connected component of a singular
-      // operator) is left out of the smoothing (dinv = 0, no couplings)
-      double dmax = 0.0;
-      for (double d : cur.diag) dmax = std::max(dmax, std::fabs(d));
-      const double dmin = 1.0e-12 * dmax;
-      std::vector<float> di(cur.n, 0.0f);
-      for (int c = 0; c < cur.n; ++c)
-        if (cur.diag[c] > dmin) di[c] = float(1.0 / cur.diag[c]);
-      auto scaled = [&](int c, size_t q, float* cs, float* cr) {
-        const int j = cur.nbr[q];
-        if (j < 0 || !(cur.diag[c] > dmin) || !(cur.diag[j] > dmin)) return false;
-        *cs = float(cur.coef[q] / cur.diag[j]);
-        *cr = float(cur.coef[q] / cur.diag[c]);
+    std::vector<AmgOp> ops(1, A);        // the operator of each level
+    std::vector<std::vector<float>> di;  // and its diagonal inverses
+    std::vector<double> dmin;
+    std::vector<AmgCsr> res;             // res[l]: level l to l + 1
+    // cs_ij = coef_ij / diag_j; a cell whose diagonal vanishes (an aggregate that is a whole
+    // connected component of a singular operator) is left out of the smoothing (dinv = 0, no
+    // couplings)
+    const auto scaled_of = [&](int l) {
+      return [&op = ops[size_t(l)], dm = dmin[size_t(l)]](int c, size_t q, double* cs) {
+        const int j = op.nbr[q];
+        if (j < 0 || !(op.diag[c] > dm) || !(op.diag[j] > dm)) return false;
+        *cs = op.coef[q] / op.diag[j];
         return true;
       };
-      if (lev == 0) {  // ELL, the solver's neighbour array
-        L.w = cur.w;
-        L.nbr = nbr_dev;
-        const size_t m = size_t(std::max(1, cur.w)) * cur.n;
-        std::vector<float> cs(m, 0.0f), cr(m, 0.0f);
-        for (int c = 0; c < cur.n; ++c)
-          for (int k = 0; k < cur.w; ++k) {
-            const size_t q = size_t(k) * cur.n + c;
-            scaled(c, q, &cs[q], &cr[q]);
-          }
-        const std::vector<AmgCoef> hcs = to_coef(cs), hcr = to_coef(cr);
-        L.cs = up(hcs);
-        L.cr = up(hcr);
-        EllOff16 o16;
-        if (off16_enabled() && ell_off16(cur.nbr.data(), cur.n, cur.w, o16)) {
-          std::vector<uint32_t> ws(size_t(o16.W) * cur.n), wr(ws.size());
-          for (size_t q = 0; q < ws.size(); ++q) {
-            const int s = o16.src[q];
-            const size_t q0 = size_t(s) * cur.n + q % size_t(cur.n);
-            const uint32_t hi = uint32_t(uint16_t(o16.d[q])) << 16;
-            ws[q] = hi | (s < 0 ? 0u : uint32_t(hcs[q0]));
-            wr[q] = hi | (s < 0 ? 0u : uint32_t(hcr[q0]));
-          }
-          L.hs = up(ws);
-          L.hr = up(wr);
-          for (int k = 0; k < 8; ++k) L.obase[k] = o16.base[k];
-        }
-      } else {  // the non-empty entries, sliced ELL
-        std::vector<int> rptr(size_t(cur.n) + 1, 0), col;
-        std::vector<float> cs, cr;
+    };
+    ops.reserve(size_t(cfg.max_levels));
+    for (int lev = 0;; ++lev) {
+      const AmgOp& cur = ops[size_t(lev)];
+      AmgLevelDev L;
+      L.n = cur.n;
+      double dmax = 0.0;
+      for (double d : cur.diag) dmax = std::max(dmax, std::fabs(d));
+      dmin.push_back(1.0e-12 * dmax);
+      di.emplace_back(cur.n, 0.0f);
+      for (int c = 0; c < cur.n; ++c)
+        if (cur.diag[c] > dmin.back()) di.back()[c] = float(1.0 / cur.diag[c]);
+      L.dinv = up(di.back());
+      const auto scaled = scaled_of(lev);
+      if (lev == 0) {
+        build_level0(L, cur, nbr_dev, scaled);
+      } else {  // the non-empty entries, packed rows
+        AmgCsr S;
+        S.ptr.assign(size_t(cur.n) + 1, 0);
         for (int c = 0; c < cur.n; ++c) {
           for (int k = 0; k < cur.w; ++k) {
-            float a, b;
-            if (!scaled(c, size_t(k) * cur.n + c, &a, &b)) continue;
-            col.push_back(cur.nbr[size_t(k) * cur.n + c]);
-            cs.push_back(a);
-            cr.push_back(b);
+            double a;
+            if (!scaled(c, size_t(k) * cur.n + c, &a)) continue;
+            S.col.push_back(cur.nbr[size_t(k) * cur.n + c]);
+            S.val.push_back(a);
           }
-          rptr[size_t(c) + 1] = int(col.size());
+          S.ptr[size_t(c) + 1] = int(S.col.size());
         }
-        std::vector<int> sptr, pos;
-        const size_t m = amg_sell_layout(cur.n, rptr, sptr, pos);
-        std::vector<int> scol(std::max<size_t>(1, m), 0);
-        std::vector<float> scs(std::max<size_t>(1, m), 0.0f), scr(std::max<size_t>(1, m), 0.0f);
-        for (int c = 0; c < cur.n; ++c) {  // padding: the row itself, zero coefficients
-          const int sl = c / AMG_SL, w = (sptr[sl + 1] - sptr[sl]) / AMG_SL;
-          for (int k = 0; k < w; ++k) scol[size_t(sptr[sl]) + size_t(k) * AMG_SL + c % AMG_SL] = c;
-        }
-        for (size_t q = 0; q < col.size(); ++q) {
-          scol[pos[q]] = col[q];
-          scs[pos[q]] = cs[q];
-          scr[pos[q]] = cr[q];
-        }
-        L.sptr = up(sptr);
-        L.col = up(scol);
-        L.cs = up(to_coef(scs));
-        L.cr = up(to_coef(scr));
-        nnz_.push_back(int64_t(col.size()));
-        stored_.push_back(int64_t(m));
+        std::vector<int> sptr, scol;
+        std::vector<float> scs;
+        packed(S, cur.n, sptr, scol, scs);
+        L.S.ptr = up(sptr);
+        L.S.col = up(scol);
+        L.S.val = up(to_coef(scs));
+        nnz_.push_back(int64_t(S.col.size()));
+        stored_.push_back(int64_t(scol.size()));
+        L.b = fresh<float>(size_t(cur.n) + 3);  // read four at a time by the dense product
+        L.y = fresh<float>(cur.n);
       }
-      L.dinv = up(di);
-      L.b = lev == 0 ? nullptr : fresh<float>(cur.n);
-      L.x = fresh<float>(cur.n);
-      L.r = fresh<float>(cur.n);
       sizes_.push_back(cur.n);
       const bool last = (cur.n <= cfg.coarse_max && lev > 0) || lev + 1 >= cfg.max_levels;
       if (last) {
         if (cur.n > 4096) throw std::runtime_error("multigrid: coarsest level too large for the dense solve");
-        std::vector<float> inv;
-        bool sing = false;
-        amg_dense_inverse(cur, inv, &sing);
-        inv_ = up(inv);
-        n_coarse_ = cur.n;
-        singular_ = sing;
         levels_.push_back(L);
         break;
       }
@@ -880,27 +890,47 @@ class AmgPc : public FcgPc, public FcgPc32 {
       }
       if (na * 3 > cur.n * 2 && cur.n > 16)  // stalled coarsening: every connection counts as strong
         na = amg_aggregate(cur, 0.0, agg);
-      if (lev == 0) agg0 = up(agg);
       std::vector<int> ptr, idx;
       amg_children(agg, na, ptr, idx);
-      AmgOp next = amg_galerkin(cur, agg, na, ptr, idx);
-      {
-        std::vector<int> kptr, pos;
-        const size_t m = amg_sell_layout(na, ptr, kptr, pos);
-        std::vector<int> kidx(std::max<size_t>(1, m), -1);
-        for (size_t q = 0; q < idx.size(); ++q) kidx[pos[q]] = idx[q];
-        L.kptr = up(kptr);
-        L.kidx = up(kidx);
+      if (lev == 0) {
+        L.agg = up(agg);
+        L.x = fresh<float>(cur.n);
       }
+      res.push_back(amg_restriction(cur, cfg.omega, na, ptr, idx, scaled));
+      AmgOp next = amg_galerkin(cur, agg, na, ptr, idx);
       levels_.push_back(L);
-      cur = std::move(next);
+      ops.push_back(std::move(next));
     }
-    if (levels_.size() >= 3) {  // the finest post-smoothing adds level 1's correction itself
-      levels_[1].y = fresh<float>(size_t(levels_[1].n));
-      levels_[0].agg = agg0;
-      levels_[0].yc = levels_[1].y;
+    // the dense bottom: the coarsest inverse, then the cycles of the small levels above it
+    bottom_ = int(levels_.size()) - 1;
+    std::vector<float> M;
+    bool sing = false;
+    amg_dense_inverse(ops[size_t(bottom_)], M, &sing);
+    singular_ = sing;
+    while (bottom_ > 1 && ops[size_t(bottom_) - 1].n <= cfg.dense_max) {
+      --bottom_;
+      M = amg_fold(ops[size_t(bottom_)], res[size_t(bottom_)], M, cfg.omega, alpha_, di[size_t(bottom_)],
+                   scaled_of(bottom_));
     }
-    zpart_ = fresh<double>(size_t(x_->pass_grid(A.n)));
+    const int nd = levels_[size_t(bottom_)].n;
+    lda_ = (nd + 3) / 4 * 4;
+    std::vector<float> padded(size_t(nd) * lda_, 0.0f);
+    for (int i = 0; i < nd; ++i) std::copy(&M[size_t(i) * nd], &M[size_t(i) * nd] + nd, &padded[size_t(i) * lda_]);
+    dense_ = up(padded);
+    const auto put = [&](const AmgCsr& m, int n, AmgMat<float>& o) {
+      std::vector<int> ptr, col;
+      std::vector<float> val;
+      packed(m, n, ptr, col, val);
+      o.ptr = up(ptr);
+      o.col = up(col);
+      o.val = up(val);
+    };
+    for (int l = 0; l < bottom_; ++l) {
+      AmgLevelDev& L = levels_[size_t(l)];
+      put(res[size_t(l)], levels_[size_t(l) + 1].n, L.R);
+      if (l > 0) put(amg_transpose(res[size_t(l)], L.n), L.n, L.Q);
+    }
+    levels_[0].yc = levels_[1].y;
   }
   void destroy() {
     if (!x_) return;
@@ -911,10 +941,10 @@ class AmgPc : public FcgPc, public FcgPc32 {
   }
   ~AmgPc() override { destroy(); }
 
-  int levels() const { return int(levels_.size()); }
+  int levels() const { return int(sizes_.size()); }
   const std::vector<int>& sizes() const { return sizes_; }
   const std::vector<int64_t>& nnz() const { return nnz_; }
-  const std::vector<int64_t>& stored() const { return stored_; }  // sliced-ELL slots, padding included
+  const std::vector<int64_t>& stored() const { return stored_; }  // slots, padding included
   bool singular() const { return singular_; }
   double alpha() const { return alpha_; }
   bool aggressive() const { return aggressive_; }
@@ -940,6 +970,55 @@ class AmgPc : public FcgPc, public FcgPc32 {
   }
 
  private:
+  // level 0: the solver's neighbour array with the scaled couplings, and their compact form
+  template <class Scaled>
+  void build_level0(AmgLevelDev& L, const AmgOp& cur, const int* nbr_dev, Scaled&& scaled) {
+    L.w = cur.w;
+    L.nbr = nbr_dev;
+    const size_t m = size_t(std::max(1, cur.w)) * cur.n;
+    std::vector<float> cs(m, 0.0f), cr(m, 0.0f);
+    for (int c = 0; c < cur.n; ++c)
+      for (int k = 0; k < cur.w; ++k) {
+        const size_t q = size_t(k) * cur.n + c;
+        double a;
+        if (!scaled(c, q, &a)) continue;
+        cs[q] = float(a);
+        cr[q] = float(cur.coef[q] / cur.diag[c]);
+      }
+    const std::vector<AmgCoef> hcs = to_coef(cs), hcr = to_coef(cr);
+    L.cs = up(hcs);
+    L.cr = up(hcr);
+    EllOff16 o16;
+    if (off16_enabled() && ell_off16(cur.nbr.data(), cur.n, cur.w, o16)) {
+      std::vector<uint32_t> ws(size_t(o16.W) * cur.n), wr(ws.size());
+      for (size_t q = 0; q < ws.size(); ++q) {
+        const int s = o16.src[q];
+        const size_t q0 = size_t(s) * cur.n + q % size_t(cur.n);
+        const uint32_t hi = uint32_t(uint16_t(o16.d[q])) << 16;
+        ws[q] = hi | (s < 0 ? 0u : uint32_t(hcs[q0]));
+        wr[q] = hi | (s < 0 ? 0u : uint32_t(hcr[q0]));
+      }
+      L.hs = up(ws);
+      L.hr = up(wr);
+      for (int k = 0; k < 8; ++k) L.obase[k] = o16.base[k];
+    }
+  }
+  // a CSR matrix of n rows as packed rows
+  static void packed(const AmgCsr& m, int n, std::vector<int>& ptr, std::vector<int>& col, std::vector<float>& val) {
+    ptr.assign(size_t(n) + 1, 0);
+    for (int r = 0; r < n; ++r) ptr[size_t(r) + 1] = ptr[r] + (m.ptr[r + 1] - m.ptr[r] + AMG_UN - 1) / AMG_UN;
+    if (int64_t(ptr[n]) * AMG_UN > INT32_MAX) throw std::runtime_error("multigrid: a level's matrix exceeds 2^31 entries");
+    const size_t size = std::max<size_t>(AMG_UN, size_t(ptr[n]) * AMG_UN);
+    col.assign(size, 0);
+    val.assign(size, 0.0f);
+    for (int r = 0; r < n; ++r) {
+      const int first = m.ptr[r + 1] > m.ptr[r] ? m.col[size_t(m.ptr[r])] : 0;
+      for (int k = ptr[r] * AMG_UN, q = m.ptr[r]; k < ptr[r + 1] * AMG_UN; ++k, ++q) {
+        col[size_t(k)] = q < m.ptr[r + 1] ? m.col[size_t(q)] : first;
+        val[size_t(k)] = q < m.ptr[r + 1] ? float(m.val[size_t(q)]) : 0.0f;
+      }
+    }
+  }
   template <class T>
   T* up(const std::vector<T>& v) {
     T* p = x_->template alloc<T>(std::max<size_t>(1, v.size()));
@@ -964,47 +1043,28 @@ class AmgPc : public FcgPc, public FcgPc32 {
              double* out_part, int mode) {
     X& xx = *x_;
     const float om = float(cfg_.omega), al = float(alpha_);
-    const int nl = int(levels_.size());
     const AmgLevelDev& L0 = levels_[0];
-    if (sc)
-      with_width(L0.w, [&](auto wc) {
-        xx.tbegin(K_MG_DOWN);
-        xx.template pass<1, 1>(L0.n, amgk::Down0<T, decltype(wc)::value>{L0, r, sc, mode, k, om}, rr_part, rr_g,
-                               zpart_);
-        xx.tend(K_MG_DOWN);
-      });
-    else
-      xx.for_each(L0.n, amgk::Down0F<T>{L0, r, om});
-    for (int l = 1; l < nl; ++l) {
-      const AmgLevelDev& F = levels_[l - 1];
-      const AmgLevelDev& C = levels_[l];
-      if (C.n >= amgk::AMG_SMALL_ROWS) {
-        xx.for_each(C.n, amgk::Restrict<1>{F.kptr, F.kidx, F.r, C.b, sc, mode});
-        if (l < nl - 1) xx.for_each(C.n, amgk::DownC<1>{C, sc, mode, om});
-      } else {
-        xx.for_each(C.n * 4, amgk::Restrict<4>{F.kptr, F.kidx, F.r, C.b, sc, mode});
-        if (l < nl - 1) xx.for_each(C.n * 4, amgk::DownC<4>{C, sc, mode, om});
-      }
+    const int n1 = levels_[1].n;
+    float* b1 = levels_[1].b;
+    xx.tbegin(K_MG_DOWN);
+    xx.template pass<1, 0>(n1 * amgk::AMG_GR, amgk::Restrict0<T>{L0.R, r, b1, sc, mode, k}, rr_part, rr_g,
+                           (double*)nullptr);
+    xx.tend(K_MG_DOWN);
+    for (int l = 1; l < bottom_; ++l) {
+      const AmgLevelDev &C = levels_[size_t(l)], &N = levels_[size_t(l) + 1];
+      xx.for_each(N.n * amgk::AMG_GR, amgk::RestrictS{C.R, C.b, N.b, sc, mode});
     }
-    {
-      const AmgLevelDev& F = levels_[nl - 2];
-      xx.for_each(n_coarse_ * amgk::AMG_GC,
-                  amgk::Coarsest{n_coarse_, inv_, levels_[nl - 1].b, F.kptr, F.kidx, F.x, sc, mode, al});
+    const AmgLevelDev& B = levels_[size_t(bottom_)];
+    xx.for_each(B.n * amgk::AMG_GC, amgk::DenseS{lda_, dense_, B.b, B.y, sc, mode});
+    for (int l = bottom_ - 1; l >= 1; --l) {
+      const AmgLevelDev& C = levels_[size_t(l)];
+      xx.for_each(C.n * amgk::AMG_GU, amgk::UpS{C, levels_[size_t(l) + 1].y, sc, mode, om, al});
     }
-    for (int l = nl - 2; l >= 1; --l) {
-      const AmgLevelDev& C = levels_[l];
-      const AmgLevelDev& F = levels_[l - 1];
-      float* yout = (l == 1 && L0.agg) ? C.y : nullptr;
-      if (C.n >= amgk::AMG_SMALL_ROWS)
-        xx.for_each(C.n, amgk::UpC<1>{C, F.kptr, F.kidx, F.x, sc, mode, om, al, yout});
-      else
-        xx.for_each(C.n * 4, amgk::UpC<4>{C, F.kptr, F.kidx, F.x, sc, mode, om, al, yout});
-    }
-    if (L0.agg) xx.for_each(L0.n, amgk::Prolong0{L0, sc, mode, al});
+    xx.for_each(L0.n, amgk::Prolong0<T>{L0, r, sc, mode, om, al});
     if (sc)
       with_width(L0.w, [&](auto wc) {
         xx.tbegin(K_MG_UP);
-        xx.template pass<1, 5>(L0.n, amgk::Up0<T, decltype(wc)::value>{L0, r, rold, z, zs, sc, mode, om, al}, nullptr,
+        xx.template pass<0, 5>(L0.n, amgk::Up0<T, decltype(wc)::value>{L0, r, rold, z, zs, sc, mode, om, al}, nullptr,
                                0, out_part);
         xx.tend(K_MG_UP);
       });
@@ -1018,12 +1078,11 @@ class AmgPc : public FcgPc, public FcgPc32 {
   std::vector<int> sizes_;
   std::vector<int64_t> nnz_, stored_;
   std::vector<void*> owned_;
-  float* inv_ = nullptr;
+  float* dense_ = nullptr;  // the bottom's matrix, rows padded to lda_
+  int lda_ = 0, bottom_ = 1;
   double alpha_ = 1.5;
   bool aggressive_ = false;
-  int n_coarse_ = 0;
   bool singular_ = false;
-  double* zpart_ = nullptr;
 };
 
 }  // namespace dm

@@ -131,10 +131,12 @@ template <int NIN, int NOUT, class F>
 __global__ void __launch_bounds__(PBLOCK) k_pass(int n, int chunk, F f, const double* in_part, int in_g,
                                                  double* out_part, int tile) {
   Red<NIN> tot = red_identity<NIN, false>();
-  for (int q = threadIdx.x; q < in_g; q += PBLOCK)
+  if constexpr (NIN > 0) {
+    for (int q = threadIdx.x; q < in_g; q += PBLOCK)
 #pragma unroll
-    for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
-  tot = block_reduce<NIN, false, PBLOCK>(tot);
+      for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
+    tot = block_reduce<NIN, false, PBLOCK>(tot);
+  }
   const int b = xcd_block(gridDim.x);
   typename F::Scal sc;
   if (!f.setup(tot, b == 0 && threadIdx.x == 0, sc)) return;  // uniform across the grid
@@ -170,10 +172,12 @@ __global__ void __launch_bounds__(PBLOCK) k_pass(int n, int chunk, F f, const do
       for (int k = 0; k < NOUT; ++k) acc.v[k] = acc.v[k] + v.v[k];
     }
   }
-  acc = block_reduce<NOUT, false, PBLOCK>(acc);
-  if (threadIdx.x == 0)
+  if constexpr (NOUT > 0) {
+    acc = block_reduce<NOUT, false, PBLOCK>(acc);
+    if (threadIdx.x == 0)
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) out_part[size_t(k) * gridDim.x + b] = acc.v[k];
+      for (int k = 0; k < NOUT; ++k) out_part[size_t(k) * gridDim.x + b] = acc.v[k];
+  }
 }
 
 template <class T>

@@ -241,7 +241,7 @@ class SolverT {
   // relative residual reduction of one FP32 sweep (DOPAMINE_MIXED_TAU overrides, for tuning)
   // Multigrid set-up: AmgCfg's defaults; DOPAMINE_AMG_THETA / _THETA0 / _ALPHA / _COARSE override
   // the strength thresholds (all levels / the first), the coarse-correction scaling and the
-  // densely solved size.
+  // densely solved size; _DENSE the size up to which levels are folded into it.
   static AmgCfg amg_cfg() {
     AmgCfg c;
     if (const char* e = std::getenv("DOPAMINE_AMG_THETA")) c.theta = std::atof(e);
@@ -250,6 +250,7 @@ class SolverT {
     if (const char* e = std::getenv("DOPAMINE_AMG_ALPHA_AGGR")) c.alpha_aggr = std::atof(e);
     if (const char* e = std::getenv("DOPAMINE_AMG_OMEGA")) c.omega = std::atof(e);
     if (const char* e = std::getenv("DOPAMINE_AMG_COARSE")) c.coarse_max = std::max(1, std::atoi(e));
+    if (const char* e = std::getenv("DOPAMINE_AMG_DENSE")) c.dense_max = std::atoi(e);
     return c;
   }
   static double mixed_tau() {

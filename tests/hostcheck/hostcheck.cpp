@@ -139,6 +139,13 @@ int hc_ell_off16(int n, int w, const int* nbr, int* base, int16_t* d, int* src) 
   std::copy(o.src.begin(), o.src.end(), src);
   return o.W;
 }
+// Size up to which levels are folded into the cycle's dense bottom (AmgCfg::dense_max; negative:
+// the product's).
+static int g_dense_max = -1;
+void hc_amg_dense_max(int m) { g_dense_max = m; }
+static void layout(dm::AmgCfg& c) {
+  if (g_dense_max >= 0) c.dense_max = g_dense_max;
+}
 int hc_amg_solve(int n, int w, const int* nbr, const double* coef, const double* diag, const double* b, double* xv,
                  double rtol, double atol, int maxit, int nullspace, int mixed, const double cfg[5], int* its,
                  double* resid, int* info) {
@@ -156,6 +163,7 @@ int hc_amg_solve(int n, int w, const int* nbr, const double* coef, const double*
     c.alpha = cfg[2];
     c.coarse_max = int(cfg[3]);
     c.theta0 = cfg[4];  // < 0: no aggressive first coarsening
+    layout(c);
     dm::AmgPc<dm::HostExec> amg;
     amg.build(&ex, op, nbr, c);
     info[0] = amg.levels();
@@ -207,6 +215,7 @@ int hc_amg_vcycle(int n, int w, const int* nbr, const double* coef, const double
     c.alpha = cfg[2];
     c.coarse_max = int(cfg[3]);
     c.theta0 = cfg[4];
+    layout(c);
     std::vector<int> agg;
     dm::amg_aggregate(op, c.theta, agg);
     std::copy(agg.begin(), agg.end(), agg_out);
