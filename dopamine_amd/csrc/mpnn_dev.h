@@ -31,7 +31,9 @@ namespace mp {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int NCH = 32;
 // flat parameter vector: Wa0 (32x3), Wb0 (32x3), b0, Wa1 (32x32), Wb1, b1, Wa2, Wb2, b2, wo
@@ -542,133 +544,208 @@ struct GradO {
   }
 };
 
-// top layer: ga = go wo (1 - h3^2)
+// top layer: ga = go wo (1 - h3^2), four channels per item
 struct GaTop {
   const float* go;
   const __bf16 *h3, *wo;
   float* ga;
-  DM_DEV void operator()(int c) const {
+  DM_DEV void operator()(int e) const {
+    const int c = e >> 3, i = (e & 7) * 4;
     const float g = go[c];
-    for (int i = 0; i < NCH; ++i) {
-      const float h = fl(h3[size_t(c) * NCH + i]);
-      ga[size_t(c) * NCH + i] = (g * fl(wo[i])) * (1.0f - h * h);
-    }
+    const bf16x4 h = *reinterpret_cast<const bf16x4*>(h3 + size_t(c) * NCH + i);
+    f32x4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = (g * fl(wo[i + k])) * (1.0f - fl(h[k]) * fl(h[k]));
+    *reinterpret_cast<f32x4*>(ga + size_t(c) * NCH + i) = o;
   }
 };
 
-// t = ga Wb, u = ga Wa (rows of the bfloat16 weights, layer l = 1, 2)
-struct BackTU {
-  const float* ga;
-  const __bf16* Wl;  // [32][64]
-  float *t, *u;
-  DM_DEV void operator()(int c) const {
-    float g[NCH];
-    for (int i = 0; i < NCH; ++i) g[i] = ga[size_t(c) * NCH + i];
-    for (int k = 0; k < NCH; ++k) {
-      float su = 0.0f, st = 0.0f;
-      for (int i = 0; i < NCH; ++i) {
-        su = su + g[i] * fl(Wl[i * 64 + k]);
-        st = st + g[i] * fl(Wl[i * 64 + 32 + k]);
+// One layer back (l = 1, 2): gh = ga Wa + (sum_j a_cj ga_j) Wb (the neighbour sum first, so nothing
+// but ga is gathered), then ga of the layer below = gh (1 - h^2), h that layer's output (the first
+// 32 inputs saved by the layer above). A wave takes 32 cells: lane (cell, half) holds 16 of the
+// cell's channels and of its neighbour sum, and the two 32 x 32 products run on the FP32 matrix
+// instructions (v_mfma_f32_32x32x2_f32, the weights' bfloat16 values exact in FP32). Bound by
+// memory: ga read (the gathers hit L2), h read, ga written. On 131,072 cells it replaces two
+// kernels (125 us and 79 us, a lane per cell striding 128 bytes) by one of 23 us.
+template <int WC>
+__global__ void __launch_bounds__(TBLOCK) k_back(int ntiles, Graph G, const float* ga, const __bf16* Wl,
+                                                 const __bf16* xs, float* gout) {
+  const int lane = threadIdx.x & 63, half = lane >> 5, row = lane & 31;
+  float wa[16], wb[16];  // A operands: row = output channel, K step s = input channel 16 half + s
+#pragma unroll
+  for (int s = 0; s < 16; ++s) {
+    wa[s] = fl(Wl[(16 * half + s) * 64 + row]);
+    wb[s] = fl(Wl[(16 * half + s) * 64 + 32 + row]);
+  }
+  const int nw = gridDim.x * (TBLOCK / 64);
+  for (int t = xcd_block(gridDim.x) * (TBLOCK / 64) + int(threadIdx.x >> 6); t < ntiles; t += nw) {
+    const int j = t * 32 + row;
+    const bool ok = j < G.n;
+    const int jc = ok ? j : G.n - 1;
+    f32x4 own[4], m[4];
+    const f32x4* gr = reinterpret_cast<const f32x4*>(ga + size_t(jc) * NCH + 16 * half);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      own[q] = gr[q];
+      m[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const auto add = [&](int nb, float av) {
+      const f32x4* nr = reinterpret_cast<const f32x4*>(ga + size_t(nb) * NCH + 16 * half);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = nr[q];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[q][e] = m[q][e] + av * v[e];
       }
-      u[size_t(c) * NCH + k] = su;
-      t[size_t(c) * NCH + k] = st;
+    };
+    if constexpr (WC > 0) {
+      int nb[WC];
+      float av[WC];
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) slot(G, kk, jc, nb[kk], av[kk]);
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) add(nb[kk], av[kk]);
+    } else {
+      for (int kk = 0; kk < G.w; ++kk) {
+        int nb;
+        float av;
+        slot(G, kk, jc, nb, av);
+        add(nb, av);
+      }
+    }
+    bf16x4 h[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      h[g] = *reinterpret_cast<const bf16x4*>(xs + size_t(jc) * 64 + 8 * g + 4 * half);
+    f32x16 d = {};
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      d = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[s], own[s >> 2][s & 3], d, 0, 0, 0);
+      d = __builtin_amdgcn_mfma_f32_32x32x2f32(wb[s], m[s >> 2][s & 3], d, 0, 0, 0);
+    }
+    if (!ok) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {  // D[v]: output channel 8 (v / 4) + 4 half + v % 4
+      f32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = d[4 * g + e] * (1.0f - fl(h[g][e]) * fl(h[g][e]));
+      *reinterpret_cast<f32x4*>(gout + size_t(j) * NCH + 8 * g + 4 * half) = o;
     }
   }
-};
+}
 
-// gh = u + sum_j a_cj t_j; ga of the layer below = gh (1 - h^2), h = that layer's output
-// (the first 32 inputs saved by the layer above)
-struct BackGh {
-  Graph G;
-  const float *t, *u;
-  const __bf16* xs;  // [n][64]: h in the first 32
-  float* ga;
-  DM_DEV void operator()(int c) const {
-    float gh[NCH];
-    for (int k = 0; k < NCH; ++k) gh[k] = 0.0f;
-    for (int kk = 0; kk < G.w; ++kk) {
-      const size_t i = size_t(kk) * G.n + c;
-      const int j = G.nbr[i];
-      if (j < 0) continue;
-      const float av = G.a[i];
-      for (int k = 0; k < NCH; ++k) gh[k] = gh[k] + av * t[size_t(j) * NCH + k];
-    }
-    for (int k = 0; k < NCH; ++k) {
-      const float h = fl(xs[size_t(c) * 64 + k]);
-      ga[size_t(c) * NCH + k] = (u[size_t(c) * NCH + k] + gh[k]) * (1.0f - h * h);
-    }
-  }
-};
-
-// Weight gradients of layer l: G[i][k] = sum_c ga[c][i] X[c][k] (X = saved inputs, row stride
-// XS, K used columns), bias sum_c ga[c][i], and for the top layer sum_c go_c h3[c][i]. Cells
-// are staged 32 at a time in LDS; block partials in FP64, layout [block][NPARAM].
-template <int K>
-__global__ void __launch_bounds__(256) k_wgrad(int n, int chunk, const float* ga, const __bf16* X, int XS, int layer,
-                                               const float* go, const __bf16* h3, double* part) {
-  constexpr int NPT = K / 8;  // outputs per thread (32 K / 256)
-  __shared__ float sga[32][NCH + 1];
-  __shared__ float sx[32][K + 1];
-  __shared__ float sgo[32];
-  const int b = blockIdx.x, t = threadIdx.x;
+// Weight gradients of layer l: G[i][k] = sum_c ga[c][i] X[c][k] (X = saved inputs, 16 KT columns),
+// bias sum_c ga[c][i], and for the top layer sum_c go_c h3[c][i]; products and sums in FP64
+// (every product of an FP32 and a bfloat16 value is exact there). The 32 x 16 KT outputs are a
+// contraction over the cells on the FP64 matrix instructions (v_mfma_f64_16x16x4_f64, four cells
+// each), operands straight from memory: a wave's lanes read whole rows. Each wave takes 16 cells
+// at a time, the block's waves are added in order through LDS; block partials [block][NPARAM].
+// 168 us -> 23 us for KT = 4 on 131,072 cells (33 MB read).
+constexpr int WGBLOCK = 512;
+template <int KT>
+__global__ void __launch_bounds__(WGBLOCK) k_wgrad(int n, int chunk, const float* ga, const __bf16* X, int layer,
+                                                   const float* go, const __bf16* h3, double* part) {
+  constexpr int K = 16 * KT;
+  __shared__ double sh[NCH * K + 2 * NCH];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, col = lane & 15, sub = lane >> 4;
   const int lo = b * chunk, hi = min(n, lo + chunk);
-  double acc[NPT];
+  f64x4 acc[2][KT];
+  double bs[2] = {0.0, 0.0}, ws[2] = {0.0, 0.0};
 #pragma unroll
-  for (int e = 0; e < NPT; ++e) acc[e] = 0.0;
-  double bacc = 0.0, wacc = 0.0;
-  const int o0 = t * NPT, oi = o0 / K, ok0 = o0 % K;
-  for (int c0 = lo; c0 < hi; c0 += 32) {
-    const int m = min(32, hi - c0);
-    for (int e = t; e < 32 * NCH; e += 256) {
-      const int cc = e / NCH, i = e % NCH;
-      sga[cc][i] = cc < m ? ga[size_t(c0 + cc) * NCH + i] : 0.0f;
-    }
-    for (int e = t; e < 32 * K; e += 256) {
-      const int cc = e / K, k = e % K;
-      sx[cc][k] = cc < m ? fl(X[size_t(c0 + cc) * XS + k]) : 0.0f;
-    }
-    if (t < 32) sgo[t] = (go && t < m) ? go[c0 + t] : 0.0f;
-    __syncthreads();
-    for (int cc = 0; cc < m; ++cc) {
-      const double gi = sga[cc][oi];
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int e = 0; e < NPT; ++e) acc[e] = acc[e] + gi * double(sx[cc][ok0 + e]);
+    for (int t = 0; t < KT; ++t) acc[a][t] = f64x4{0.0, 0.0, 0.0, 0.0};
+  for (int c0 = lo + 16 * w; c0 < hi; c0 += 16 * (WGBLOCK / 64)) {
+    float av[4][2], xv[4][KT], gv[4], hv[4][2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = c0 + 4 * q + sub;
+      const bool ok = c < hi;
+      const size_t cc = size_t(ok ? c : hi - 1);
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const float v = ga[cc * NCH + 16 * a + col];
+        av[q][a] = ok ? v : 0.0f;
+        hv[q][a] = go ? fl(h3[cc * NCH + 16 * a + col]) : 0.0f;
+      }
+      gv[q] = (go && ok) ? go[cc] : 0.0f;
+#pragma unroll
+      for (int t = 0; t < KT; ++t) xv[q][t] = fl(X[cc * K + 16 * t + col]);
     }
-    if (t < 32) {
-      for (int cc = 0; cc < m; ++cc) bacc = bacc + double(sga[cc][t]);
-      if (go)
-        for (int cc = 0; cc < m; ++cc) wacc = wacc + double(sgo[cc]) * double(fl(h3[size_t(c0 + cc) * NCH + t]));
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const double d = av[q][a];
+        bs[a] = bs[a] + d;
+        ws[a] = ws[a] + double(gv[q]) * double(hv[q][a]);
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+          acc[a][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(d, double(xv[q][t]), acc[a][t], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {  // over the four cells of a step
+    bs[a] = bs[a] + __shfl_xor(bs[a], 16, 64);
+    bs[a] = bs[a] + __shfl_xor(bs[a], 32, 64);
+    ws[a] = ws[a] + __shfl_xor(ws[a], 16, 64);
+    ws[a] = ws[a] + __shfl_xor(ws[a], 32, 64);
+  }
+  for (int q = 0; q < WGBLOCK / 64; ++q) {
+    if (w == q) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {  // D[v]: row 4 v + lane / 16, column lane % 16
+            double* o = &sh[(16 * a + 4 * v + sub) * K + 16 * t + col];
+            *o = q == 0 ? acc[a][t][v] : *o + acc[a][t][v];
+          }
+        if (sub == 0) {
+          double* o = &sh[NCH * K + 16 * a + col];
+          o[0] = q == 0 ? bs[a] : o[0] + bs[a];
+          o[NCH] = q == 0 ? ws[a] : o[NCH] + ws[a];
+        }
+      }
     }
     __syncthreads();
   }
   double* pb = part + size_t(b) * NPARAM;
   const int kin = KIN[layer];
-#pragma unroll
-  for (int e = 0; e < NPT; ++e) {
-    const int k = ok0 + e;
+  for (int e = threadIdx.x; e < NCH * K; e += WGBLOCK) {
+    const int i = e / K, k = e % K;
     if (k < kin)
-      pb[OFF_WA[layer] + oi * kin + k] = acc[e];
+      pb[OFF_WA[layer] + i * kin + k] = sh[e];
     else if (k < 2 * kin)
-      pb[OFF_WB[layer] + oi * kin + k - kin] = acc[e];
+      pb[OFF_WB[layer] + i * kin + k - kin] = sh[e];
   }
-  if (t < 32) {
-    pb[OFF_B[layer] + t] = bacc;
-    if (go) pb[OFF_WO + t] = wacc;
+  if (threadIdx.x < NCH) {
+    pb[OFF_B[layer] + threadIdx.x] = sh[NCH * K + threadIdx.x];
+    if (go) pb[OFF_WO + threadIdx.x] = sh[NCH * K + NCH + threadIdx.x];
   }
 }
 
-// gsum[p] (+)= sum over blocks of part[b][p], in block order
-struct GradReduce {
-  const double* part;
-  int nb;
-  double* gsum;
-  int accumulate;
-  DM_DEV void operator()(int p) const {
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s = s + part[size_t(b) * NPARAM + p];
+// gsum[p] (+)= sum over blocks of part[b][p]: 32 parameters a block, eight runs of the partials
+// each in block order, then the runs in order (64 us -> 4 us with 256 partials).
+constexpr int GR_RUNS = 8;
+static __global__ void __launch_bounds__(32 * GR_RUNS) k_grad_reduce(const double* part, int nb, double* gsum,
+                                                              int accumulate) {
+  __shared__ double sh[GR_RUNS][32];
+  const int p = blockIdx.x * 32 + (threadIdx.x & 31), run = threadIdx.x >> 5;
+  const int per = (nb + GR_RUNS - 1) / GR_RUNS, b0 = run * per, b1 = min(nb, b0 + per);
+  double s = 0.0;
+  if (p < NPARAM) {
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) s = s + part[size_t(b) * NPARAM + p];
+  }
+  sh[run][threadIdx.x & 31] = s;
+  __syncthreads();
+  if (run == 0 && p < NPARAM) {
+    for (int r = 1; r < GR_RUNS; ++r) s = s + sh[r][threadIdx.x];
     gsum[p] = accumulate ? gsum[p] + s : s;
   }
-};
+}
 
 // Adam (Kingma and Ba 2015, Algorithm 1) on the FP32 master parameters; g = gsum * scale.
 struct AdamStep {
@@ -764,8 +841,7 @@ class LearnedPc : public FcgPc, public CgCapture {
     for (void* q : {(void*)a_, (void*)q_, (void*)f2_, (void*)mx2_, (void*)dinv_, (void*)dbar_, (void*)W0_, (void*)W1_,
                     (void*)W2_, (void*)wo_, (void*)bias_, (void*)p_, (void*)m_, (void*)v_, (void*)gsum_, (void*)h1_,
                     (void*)h2_, (void*)s_, (void*)rrp_, (void*)zp_, (void*)samples_, (void*)x0s_, (void*)x1s_,
-                    (void*)x2s_, (void*)h3s_, (void*)z_, (void*)y_, (void*)go_, (void*)ga_, (void*)gb_, (void*)t_,
-                    (void*)u_, (void*)wpart_, (void*)lossd_, (void*)lpart_})
+                    (void*)x2s_, (void*)h3s_, (void*)z_, (void*)y_, (void*)go_, (void*)ga_, (void*)gb_, (void*)wpart_, (void*)lossd_, (void*)lpart_})
       if (q) x_->release(q);
     x_ = nullptr;
   }
@@ -850,15 +926,14 @@ class LearnedPc : public FcgPc, public CgCapture {
     forward(r, z_, true);
     x_->template pass<1, 2>(n_, LossY{A_, z_, r, y_}, nullptr, 0, lpart_);
     x_->template pass<2, 1>(n_, GradO{A_, y_, s_, dinv_, go_, lossd_ + slot}, lpart_, g_, lpart_ + 2 * size_t(g_));
-    x_->for_each(n_, GaTop{go_, h3s_, wo_, ga_});
-    wgrad<64>(ga_, x2s_, 64, 2, go_, h3s_);
-    x_->for_each(n_, BackTU{ga_, W2_, t_, u_});
-    x_->for_each(n_, BackGh{G_, t_, u_, x2s_, gb_});
-    wgrad<64>(gb_, x1s_, 64, 1, nullptr, nullptr);
-    x_->for_each(n_, BackTU{gb_, W1_, t_, u_});
-    x_->for_each(n_, BackGh{G_, t_, u_, x1s_, ga_});
-    wgrad<8>(ga_, x0s_, 16, 0, nullptr, nullptr);
-    x_->for_each(NPARAM, GradReduce{wpart_, wgrid(), gsum_, accumulate ? 1 : 0});
+    x_->for_each(n_ * 8, GaTop{go_, h3s_, wo_, ga_});
+    wgrad<4>(ga_, x2s_, 2, go_, h3s_);
+    back(ga_, W2_, x2s_, gb_);
+    wgrad<4>(gb_, x1s_, 1, nullptr, nullptr);
+    back(gb_, W1_, x1s_, ga_);
+    wgrad<1>(ga_, x0s_, 0, nullptr, nullptr);
+    x_->launch(k_grad_reduce, (NPARAM + 31) / 32, 32 * GR_RUNS, (const double*)wpart_, wgrid(), gsum_,
+               accumulate ? 1 : 0);
   }
   void gradient(double* host) { x_->download(host, gsum_, NPARAM); }
   double loss(int slot) {
@@ -908,10 +983,14 @@ class LearnedPc : public FcgPc, public CgCapture {
   static int batch_cap() { return 16; }
 
   int wgrid() const { return std::max(1, std::min(256, (n_ + 255) / 256)); }
-  template <int K>
-  void wgrad(const float* ga, const __bf16* X, int XS, int layer, const float* go, const __bf16* h3) {
+  template <int KT>
+  void wgrad(const float* ga, const __bf16* X, int layer, const float* go, const __bf16* h3) {
     const int gb = wgrid(), chunk = (n_ + gb - 1) / gb;
-    x_->launch(k_wgrad<K>, gb, 256, n_, chunk, ga, X, XS, layer, go, h3, wpart_);
+    x_->launch(k_wgrad<KT>, gb, WGBLOCK, n_, chunk, ga, X, layer, go, h3, wpart_);
+  }
+  void back(const float* ga, const __bf16* Wl, const __bf16* xs, float* gout) {
+    const int nt = (n_ + 31) / 32, g = std::max(1, std::min(TGRID_BIG, (nt + 3) / 4));
+    by_width(G_.w, [&](auto wc) { x_->launch(k_back<decltype(wc)::value>, g, TBLOCK, nt, G_, ga, Wl, xs, gout); });
   }
   void pack() {
     x_->for_each(Pack::count(), Pack{p_, W0_, W1_, W2_, wo_, bias_});
@@ -928,8 +1007,6 @@ class LearnedPc : public FcgPc, public CgCapture {
     go_ = x_->alloc<float>(n);
     ga_ = x_->alloc<float>(n * NCH);
     gb_ = x_->alloc<float>(n * NCH);
-    t_ = x_->alloc<float>(n * NCH);
-    u_ = x_->alloc<float>(n * NCH);
     wpart_ = x_->alloc<double>(size_t(wgrid()) * NPARAM);
     lossd_ = x_->alloc<double>(size_t(LOSS_SLOTS_STEPS) * batch_cap());
     lpart_ = x_->alloc<double>(size_t(3) * g_);
@@ -967,7 +1044,7 @@ class LearnedPc : public FcgPc, public CgCapture {
   // training buffers
   __bf16 *x0s_ = nullptr, *x1s_ = nullptr, *x2s_ = nullptr, *h3s_ = nullptr;
   double *z_ = nullptr, *y_ = nullptr, *wpart_ = nullptr, *lossd_ = nullptr, *lpart_ = nullptr;
-  float *go_ = nullptr, *ga_ = nullptr, *gb_ = nullptr, *t_ = nullptr, *u_ = nullptr;
+  float *go_ = nullptr, *ga_ = nullptr, *gb_ = nullptr;
 };
 
 struct LearnCfg {
