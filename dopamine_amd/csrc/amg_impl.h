@@ -464,17 +464,18 @@ enum Mode { OUTER = 0, INNER = 1 };
 // else the kernel has issued. Level 0's kernels test it first (a pass after convergence returns at
 // once); the coarse levels' kernels, where a dependent load costs more than the work, compute
 // first and let it decide the stores.
+DM_INLINE bool gated(const cgk::Head& h, int mode) { return (h.done | (mode == INNER ? h.inner_done : 0)) != 0; }
 DM_INLINE bool gated(const CgScalars* sc, int mode) {
   if (!sc) return false;
   const int d = sc->done, e = sc->inner_done;
   return (d | (mode == INNER ? e : 0)) != 0;
 }
 
-DM_INLINE bool cycle_test(CgScalars* sc, int mode, int k, double rr, bool leader) {
+DM_INLINE bool cycle_test(CgScalars* sc, const cgk::Head& h, int mode, int k, double rr, bool leader) {
   if (!sc) return true;  // a cycle outside a solve
-  if (gated(sc, mode)) return false;
+  if (gated(h, mode)) return false;
   if (mode == OUTER) {
-    const int fin = (sqrt(rr) <= sc->ttol) ? 1 : (k >= sc->maxit ? 2 : 0);
+    const int fin = (sqrt(rr) <= h.ttol) ? 1 : (k >= h.maxit ? 2 : 0);
     if (leader) {
       sc->its = k;
       sc->rr = rr;
@@ -482,7 +483,7 @@ DM_INLINE bool cycle_test(CgScalars* sc, int mode, int k, double rr, bool leader
     }
     return fin == 0;
   }
-  if (k > 0 && (rr <= sc->inner_tol2 || sc->its + k >= sc->maxit)) {
+  if (k > 0 && (rr <= h.inner_tol2 || h.its + k >= h.maxit)) {
     if (leader) {
       sc->inner_done = 1;
       sc->inner_its = k;
@@ -632,9 +633,9 @@ struct RowGroup {
     return s;
   }
 };
-// (R x)_r by the G lanes of a group
-template <int G, class T>
-DM_INLINE float row_dot(const AmgMat<float>& m, const T* x, int r, int lane, int st) {
+// this lane's part of (R x)_r
+template <class T>
+DM_INLINE float row_part(const AmgMat<float>& m, const T* x, int r, int lane, int st) {
   const int q0 = m.ptr[r], ng = m.ptr[r + 1] - q0;
   float s = 0.0f;
   for (int g = lane; g < ng; g += st) {
@@ -642,7 +643,7 @@ DM_INLINE float row_dot(const AmgMat<float>& m, const T* x, int r, int lane, int
     c.load(m, q0, g, ng);
     s = s + c.dot(x);
   }
-  return group_sum<G>(s);
+  return s;
 }
 
 // A coarse level on the way down: the next level's right-hand side b_next = R b.
@@ -656,7 +657,7 @@ struct RestrictS {
     int lane, st;
     if (!group_lane<AMG_GR>(t, &lane, &st)) return;
     const bool off = gated(sc, mode);
-    const float s = row_dot<AMG_GR>(R, b, t / AMG_GR, lane, st);
+    const float s = group_sum<AMG_GR>(row_part(R, b, t / AMG_GR, lane, st));
     if (lane == 0 && !off) bn[t / AMG_GR] = s;
   }
 };
@@ -667,22 +668,28 @@ struct RestrictS {
 // 17.6 us on 786,432; at 7.9 million (HBM-bound) 93 us for 92 us.
 template <class T>
 struct Restrict0 {
-  static constexpr int kSlots = 1;
+  static constexpr bool kPre = true;
   AmgMat<float> R;
   const T* b;
   float* bn;
   CgScalars* sc;
   int mode, k;
   using Scal = cgk::NoScal;
-  DM_HD bool setup(const Red<1>& t, bool leader, Scal&) const { return cycle_test(sc, mode, k, t.v[0], leader); }
-  DM_HD Red<0> run(int lo, int hi, int t, int nt, const Scal&) const {
-    for (int q = lo + t; q < hi; q += nt) {
-      int lane, st;
-      if (!group_lane<AMG_GR>(q, &lane, &st)) continue;
-      const float s = row_dot<AMG_GR>(R, b, q / AMG_GR, lane, st);
-      if (lane == 0) bn[q / AMG_GR] = s;
-    }
-    return Red<0>{};
+  struct Pre {
+    float s;
+  };
+  DM_HD cgk::Head head() const { return sc ? cgk::read_head(sc, 0) : cgk::Head{}; }
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal&, const cgk::Head& h) const {
+    return cycle_test(sc, h, mode, k, t.v[0], leader);
+  }
+  DM_HD Pre load(int q) const {
+    int lane, st;
+    if (!group_lane<AMG_GR>(q, &lane, &st)) return Pre{0.0f};
+    return Pre{row_part(R, b, q / AMG_GR, lane, st)};
+  }
+  DM_HD void apply(int q, const Pre& o, const Scal&, Red<0>&) const {
+    const float s = group_sum<AMG_GR>(o.s);
+    if (q % AMG_GR == 0) bn[q / AMG_GR] = s;
   }
 };
 
@@ -755,7 +762,7 @@ struct DenseS {
 // sweeps, which form z.r_old from it)
 template <class T, int WC = 0>
 struct Up0 {
-  static constexpr int kSlots = WC;
+  static constexpr bool kPre = WC > 0;
   AmgLevelDev L;
   const T *r, *rold;  // rold: the v of the partials
   T* z;  // z[c * zs]
@@ -764,7 +771,13 @@ struct Up0 {
   int mode;
   float omega, al;
   using Scal = cgk::NoScal;
+  struct Pre {
+    float h[WC > 0 ? WC : 1], xj[WC > 0 ? WC : 1], x, di;
+    T r, ro;
+  };
+  DM_HD cgk::Head head() const { return cgk::read_head(sc, 0); }
   DM_HD bool setup(const Red<0>&, bool, Scal&) const { return !gated(sc, mode); }
+  DM_HD bool setup(const Red<0>&, bool, Scal&, const cgk::Head& h) const { return !gated(h, mode); }
   DM_HD Red<5> operator()(int c, const Scal&) const {
     const float y = up_cell(L, r, omega, al, c);
     const T zc = T(y);
@@ -778,32 +791,33 @@ struct Up0 {
     o.v[4] = ro;
     return o;
   }
-  DM_HD Red<5> run(int lo, int hi, int t, int nt, const Scal&) const {
-    Red<5> acc = red_identity<5, false>();
-    for (int c = lo + t; c < hi; c += nt) {
-      int jj[WC > 0 ? WC : 1];
-      float h[WC > 0 ? WC : 1], xj[WC > 0 ? WC : 1];
-      if (L.hr)
-        slots0p<WC>(L, L.hr, c, jj, h);
-      else
-        slots0<WC>(L, L.cr, c, jj, h);
+  DM_HD Pre load(int c) const {
+    Pre o;
+    int jj[WC > 0 ? WC : 1];
+    if (L.hr)
+      slots0p<WC>(L, L.hr, c, jj, o.h);
+    else
+      slots0<WC>(L, L.cr, c, jj, o.h);
+    o.x = L.x[c];
+    o.di = L.dinv[c];
+    o.r = r[c];
+    o.ro = rold[c];
 #pragma unroll
-      for (int kk = 0; kk < WC; ++kk) xj[kk] = L.x[jj[kk]];
-      const float xc = L.x[c];
-      const float bc = float(r[c]);
-      float s = 0.0f;
+    for (int kk = 0; kk < WC; ++kk) o.xj[kk] = L.x[jj[kk]];
+    return o;
+  }
+  DM_HD void apply(int c, const Pre& o, const Scal&, Red<5>& acc) const {
+    float s = 0.0f;
 #pragma unroll
-      for (int kk = 0; kk < WC; ++kk) s = s + h[kk] * xj[kk];
-      const T zc = T(xc + omega * (L.dinv[c] * bc - xc + s));
-      z[size_t(c) * zs] = zc;
-      const double rc = double(r[c]), ro = double(rold[c]), zd = double(zc);
-      acc.v[0] = acc.v[0] + zd * rc;
-      acc.v[1] = acc.v[1] + zd * ro;
-      acc.v[2] = acc.v[2] + zd;
-      acc.v[3] = acc.v[3] + rc;
-      acc.v[4] = acc.v[4] + ro;
-    }
-    return acc;
+    for (int kk = 0; kk < WC; ++kk) s = s + o.h[kk] * o.xj[kk];
+    const T zc = T(o.x + omega * (o.di * float(o.r) - o.x + s));
+    z[size_t(c) * zs] = zc;
+    const double rc = double(o.r), ro = double(o.ro), zd = double(zc);
+    acc.v[0] = acc.v[0] + zd * rc;
+    acc.v[1] = acc.v[1] + zd * ro;
+    acc.v[2] = acc.v[2] + zd;
+    acc.v[3] = acc.v[3] + rc;
+    acc.v[4] = acc.v[4] + ro;
   }
 };
 

@@ -244,6 +244,17 @@ namespace cgk {
 
 struct NoScal {};
 
+// What a pass's setup() reads of the solve's scalars, the histories at one index. (Read as single
+// fields: a copy of the whole struct, indexed at run time, would live in scratch memory.)
+struct Head {
+  int done, inner_done, its, maxit, nullspace;
+  double ttol, inner_tol2, rz, gamma, alpha, alpha32;
+};
+DM_INLINE Head read_head(const CgScalars* s, int at) {
+  return Head{s->done, s->inner_done, s->its, s->maxit, s->nullspace, s->ttol, s->inner_tol2, s->rz_hist[at],
+              s->gamma_hist[at], s->alpha_hist[at], s->alpha32};
+}
+
 // b' = finite(b), x scrubbed; partial: sum b'
 struct SumB {
   const double* b;
@@ -321,7 +332,12 @@ struct Z0 {
 // ||r_k|| <= ttol (KSPCG tests after each update, and once before the first), the projected
 // r.z = r.z - mean(z) sum r, and beta = (r.z)_k / (r.z)_(k-1). Then p = (z - mean z) + beta p_old
 // for this row and, recomputed on the fly, for its neighbours; q = A p; partial p.q.
-struct Dir {
+// The batched form (WC > 0, used on the device and by the host check) reads WC operator slots
+// branch-free: a slot past the operator's width or without a neighbour reads the cell itself and
+// has a zero coefficient, which subtracts an exact zero.
+template <int WC>
+struct DirT {
+  static constexpr bool kPre = WC > 0;
   EllOp A;
   const double *z, *pold;
   double *pnew, *q;
@@ -330,12 +346,17 @@ struct Dir {
   struct Scal {
     double zm, beta;
   };
-  DM_HD bool setup(const Red<4>& t, bool leader, Scal& s) const {
-    if (sc->done) return false;
+  struct Pre {
+    double cf[WC > 0 ? WC : 1], zj[WC > 0 ? WC : 1], pj[WC > 0 ? WC : 1], z, p, d;
+  };
+  DM_HD Head head() const { return read_head(sc, (k + 1) & 1); }
+  DM_HD bool setup(const Red<4>& t, bool leader, Scal& s) const { return setup(t, leader, s, head()); }
+  DM_HD bool setup(const Red<4>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done) return false;
     const double rr = t.v[0];
-    s.zm = sc->nullspace ? t.v[2] / double(A.n) : 0.0;
+    s.zm = h.nullspace ? t.v[2] / double(A.n) : 0.0;
     const double rz = t.v[1] - s.zm * t.v[3];
-    const int fin = (sqrt(rr) <= sc->ttol) ? 1 : (k >= sc->maxit ? 2 : 0);
+    const int fin = (sqrt(rr) <= h.ttol) ? 1 : (k >= h.maxit ? 2 : 0);
     if (leader) {
       sc->its = k;
       sc->rr = rr;
@@ -343,19 +364,54 @@ struct Dir {
       else sc->rz_hist[k & 1] = rz;
     }
     if (fin) return false;
-    s.beta = k == 0 ? 0.0 : rz / sc->rz_hist[(k + 1) & 1];
+    s.beta = k == 0 ? 0.0 : rz / h.rz;
     return true;
+  }
+  DM_HD double dir(double zv, double pv, const Scal& s) const {
+    return k == 0 ? (zv - s.zm) : (zv - s.zm) + s.beta * pv;
+  }
+  DM_HD Pre load(int c) const {
+    Pre o;
+    const int n = A.n, w = A.w;
+    const bool first = k == 0;
+    int jj[WC > 0 ? WC : 1];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) {
+      const bool live = kk < w;
+      const size_t q_ = size_t(live ? kk : 0) * n + c;
+      const int j = A.nbr[q_];
+      const double h = A.coef[q_];
+      jj[kk] = (live && j >= 0) ? j : c;
+      o.cf[kk] = (live && j >= 0) ? h : 0.0;
+    }
+    o.z = z[c];
+    o.p = first ? 0.0 : pold[c];
+    o.d = A.diag[c];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) {
+      o.zj[kk] = z[jj[kk]];
+      o.pj[kk] = first ? 0.0 : pold[jj[kk]];
+    }
+    return o;
+  }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<1>& acc) const {
+    const double pc = dir(o.z, o.p, s);
+    double qc = o.d * pc;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) qc = qc - o.cf[kk] * dir(o.zj[kk], o.pj[kk], s);
+    pnew[c] = pc;
+    q[c] = qc;
+    acc.v[0] = acc.v[0] + pc * qc;
   }
   DM_HD Red<1> operator()(int c, const Scal& s) const {
     const int n = A.n;
     const bool first = k == 0;
-    const double pc = first ? (z[c] - s.zm) : (z[c] - s.zm) + s.beta * pold[c];
+    const double pc = dir(z[c], first ? 0.0 : pold[c], s);
     double qc = A.diag[c] * pc;
     for (int kk = 0; kk < A.w; ++kk) {
       const int j = A.nbr[size_t(kk) * n + c];
       if (j < 0) continue;
-      const double pj = first ? (z[j] - s.zm) : (z[j] - s.zm) + s.beta * pold[j];
-      qc = qc - A.coef[size_t(kk) * n + c] * pj;
+      qc = qc - A.coef[size_t(kk) * n + c] * dir(z[j], first ? 0.0 : pold[j], s);
     }
     pnew[c] = pc;
     q[c] = qc;
@@ -368,6 +424,7 @@ struct Dir {
 // Iteration k, second pass: alpha = (r.z)_k / p.q; x += alpha p, r -= alpha q, z = D^-1 r;
 // partials r.r, r.z, sum z, sum r for the next test.
 struct Upd {
+  static constexpr bool kPre = true;
   const double *diag, *p, *q;
   double *x, *r, *z;
   CgScalars* sc;
@@ -375,23 +432,26 @@ struct Upd {
   struct Scal {
     double a;
   };
-  DM_HD bool setup(const Red<1>& t, bool, Scal& s) const {
-    if (sc->done) return false;
-    s.a = sc->rz_hist[k & 1] / t.v[0];
+  struct Pre {
+    double x, p, r, q, d;
+  };
+  DM_HD Head head() const { return read_head(sc, k & 1); }
+  DM_HD bool setup(const Red<1>& t, bool, Scal& s, const Head& h) const {
+    if (h.done) return false;
+    s.a = h.rz / t.v[0];
     return true;
   }
-  DM_HD Red<4> operator()(int c, const Scal& s) const {
-    x[c] = x[c] + s.a * p[c];
-    const double rc = r[c] - s.a * q[c];
+  DM_HD Pre load(int c) const { return Pre{x[c], p[c], r[c], q[c], diag[c]}; }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<4>& acc) const {
+    x[c] = o.x + s.a * o.p;
+    const double rc = o.r - s.a * o.q;
     r[c] = rc;
-    const double zc = rc / diag[c];
+    const double zc = rc / o.d;
     z[c] = zc;
-    Red<4> o;
-    o.v[0] = rc * rc;
-    o.v[1] = rc * zc;
-    o.v[2] = zc;
-    o.v[3] = rc;
-    return o;
+    acc.v[0] = acc.v[0] + rc * rc;
+    acc.v[1] = acc.v[1] + rc * zc;
+    acc.v[2] = acc.v[2] + zc;
+    acc.v[3] = acc.v[3] + rc;
   }
 };
 
@@ -462,19 +522,14 @@ struct W0 {
 // beta_k gamma_k / alpha_(k-1)); p = u + beta p, s = w + beta s, x += alpha p, r -= alpha s,
 // w' = A D^-1 r' with the neighbours' r' recomputed on the fly from their old r, s, w.
 // The old packed state is read from one buffer and the new one written to the other.
-// The batched form (WC > 0, used on the device) reads WC neighbour slots branch-free: a slot past
-// the operator's width or without a neighbour reads the cell's own state and has a zero
-// coefficient (chat is zero on empty slots), which subtracts an exact zero. Each thread takes U
-// cells at a time, so all their loads are issued before the first result is needed. At k = 0 the
-// state's s and p are zero (W0 writes them), so beta = 0 gives the first iteration's values.
-#ifndef DM_CG_CELLS_PER_THREAD
-#define DM_CG_CELLS_PER_THREAD 1
-#endif
-constexpr int CG_U = DM_CG_CELLS_PER_THREAD;
+// The batched form (WC > 0) reads WC neighbour slots branch-free, as DirT: a slot past the
+// operator's width or without a neighbour reads the cell's own state and has a zero coefficient
+// (chat is zero on empty slots), which subtracts an exact zero. At k = 0 the state's s and p are
+// zero (W0 writes them), so beta = 0 gives the first iteration's values.
 
 template <int WC>
 struct FusedT {
-  static constexpr int kSlots = WC;
+  static constexpr bool kPre = WC > 0;
   JacobiScaled J;
   const St4* st0;
   St4* st1;
@@ -484,13 +539,19 @@ struct FusedT {
   struct Scal {
     double um, beta, alpha;
   };
-  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s) const {
-    if (sc->done) return false;
+  struct Pre {
+    St4 o, nj[WC > 0 ? WC : 1];
+    double di, x, ch[WC > 0 ? WC : 1];
+  };
+  DM_HD Head head() const { return read_head(sc, (k + 1) & 1); }
+  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s) const { return setup(t, leader, s, head()); }
+  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done) return false;
     const double rr = t.v[0];
-    s.um = sc->nullspace ? t.v[3] / double(J.n) : 0.0;
+    s.um = h.nullspace ? t.v[3] / double(J.n) : 0.0;
     const double gamma = t.v[1] - s.um * t.v[4];
     const double delta = t.v[2] - s.um * t.v[5];
-    const int fin = (sqrt(rr) <= sc->ttol) ? 1 : (k >= sc->maxit ? 2 : 0);
+    const int fin = (sqrt(rr) <= h.ttol) ? 1 : (k >= h.maxit ? 2 : 0);
     if (fin) {
       if (leader) {
         sc->its = k;
@@ -503,8 +564,8 @@ struct FusedT {
       s.beta = 0.0;
       s.alpha = gamma / delta;
     } else {
-      s.beta = gamma / sc->gamma_hist[(k + 1) & 1];
-      s.alpha = gamma / (delta - s.beta * gamma / sc->alpha_hist[(k + 1) & 1]);
+      s.beta = gamma / h.gamma;
+      s.alpha = gamma / (delta - s.beta * gamma / h.alpha);
     }
     if (leader) {
       sc->its = k;
@@ -544,56 +605,40 @@ struct FusedT {
     st1[c] = St4{rc, sc_, wc, pc};
     return sums(rc, rc * di, wc);
   }
-  DM_HD Red<6> run(int lo, int hi, int t, int nt, const Scal& s) const {
+  DM_HD Pre load(int c) const {
+    Pre p;
     const int n = J.n, w = J.w;
-    Red<6> acc = red_identity<6, false>();
-    for (int c0 = lo + t; c0 < hi; c0 += CG_U * nt) {
-      int cc[CG_U];
-      St4 o[CG_U];
-      double di[CG_U], xo[CG_U], ch[CG_U][WC], g[CG_U][WC];
-      int jj[CG_U][WC];
+    int jj[WC > 0 ? WC : 1];
 #pragma unroll
-      for (int u = 0; u < CG_U; ++u) {
-        cc[u] = (c0 + u * nt < hi) ? c0 + u * nt : c0;
-        o[u] = st0[cc[u]];
-        di[u] = J.dinv[cc[u]];
-        xo[u] = x[cc[u]];
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) {
-          const bool live = kk < w;
-          const size_t q = size_t(live ? kk : 0) * n + cc[u];
-          const int j = J.nbr[q];
-          const double h = J.chat[q];
-          jj[u][kk] = (live && j >= 0) ? j : cc[u];
-          ch[u][kk] = live ? h : 0.0;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < CG_U; ++u)
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) {
-          const St4 nj = st0[jj[u][kk]];
-          g[u][kk] = nj.r - s.alpha * (nj.w + s.beta * nj.s);
-        }
-#pragma unroll
-      for (int u = 0; u < CG_U; ++u) {
-        const double uc = o[u].r * di[u] - s.um;
-        const double pc = uc + s.beta * o[u].p;
-        const double sc_ = o[u].w + s.beta * o[u].s;
-        const double rc = o[u].r - s.alpha * sc_;
-        double wc = rc;
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) wc = wc - ch[u][kk] * g[u][kk];
-        if (c0 + u * nt < hi) {
-          x[cc[u]] = xo[u] + s.alpha * pc;
-          st1[cc[u]] = St4{rc, sc_, wc, pc};
-          const Red<6> v = sums(rc, rc * di[u], wc);
-#pragma unroll
-          for (int q = 0; q < 6; ++q) acc.v[q] = acc.v[q] + v.v[q];
-        }
-      }
+    for (int kk = 0; kk < WC; ++kk) {
+      const bool live = kk < w;
+      const size_t q = size_t(live ? kk : 0) * n + c;
+      const int j = J.nbr[q];
+      const double h = J.chat[q];
+      jj[kk] = (live && j >= 0) ? j : c;
+      p.ch[kk] = live ? h : 0.0;
     }
-    return acc;
+    p.o = st0[c];
+    p.di = J.dinv[c];
+    p.x = x[c];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) p.nj[kk] = st0[jj[kk]];
+    return p;
+  }
+  DM_HD void apply(int c, const Pre& p, const Scal& s, Red<6>& acc) const {
+    const double uc = p.o.r * p.di - s.um;
+    const double pc = uc + s.beta * p.o.p;
+    const double sc_ = p.o.w + s.beta * p.o.s;
+    const double rc = p.o.r - s.alpha * sc_;
+    double wc = rc;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk)
+      wc = wc - p.ch[kk] * (p.nj[kk].r - s.alpha * (p.nj[kk].w + s.beta * p.nj[kk].s));
+    x[c] = p.x + s.alpha * pc;
+    st1[c] = St4{rc, sc_, wc, pc};
+    const Red<6> v = sums(rc, rc * p.di, wc);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) acc.v[q] = acc.v[q] + v.v[q];
   }
 };
 using Fused = FusedT<0>;
@@ -700,7 +745,7 @@ struct IrStart {
 // One FP32 single-reduction iteration of a sweep (as FusedT); the correction e accumulates in FP32.
 template <int WC>
 struct Fused32T {
-  static constexpr int kSlots = WC;
+  static constexpr bool kPre = WC > 0;
   JacobiScaled J;
   const St4f* st0;
   St4f* st1;
@@ -710,13 +755,19 @@ struct Fused32T {
   struct Scal {
     double um, beta, alpha;
   };
-  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s) const {
-    if (sc->done || sc->inner_done) return false;
+  struct Pre {
+    St4f o, nj[WC > 0 ? WC : 1];
+    float di, e, ch[WC > 0 ? WC : 1];
+  };
+  DM_HD Head head() const { return read_head(sc, (k + 1) & 1); }
+  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s) const { return setup(t, leader, s, head()); }
+  DM_HD bool setup(const Red<6>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done || h.inner_done) return false;
     const double rr = t.v[0];
-    s.um = sc->nullspace ? t.v[3] / double(J.n) : 0.0;
+    s.um = h.nullspace ? t.v[3] / double(J.n) : 0.0;
     const double gamma = t.v[1] - s.um * t.v[4];
     const double delta = t.v[2] - s.um * t.v[5];
-    if (k > 0 && (rr <= sc->inner_tol2 || sc->its + k >= sc->maxit)) {
+    if (k > 0 && (rr <= h.inner_tol2 || h.its + k >= h.maxit)) {
       if (leader) {
         sc->inner_done = 1;
         sc->inner_its = k;
@@ -727,8 +778,8 @@ struct Fused32T {
       s.beta = 0.0;
       s.alpha = gamma / delta;
     } else {
-      s.beta = gamma / sc->gamma_hist[(k + 1) & 1];
-      s.alpha = gamma / (delta - s.beta * gamma / sc->alpha_hist[(k + 1) & 1]);
+      s.beta = gamma / h.gamma;
+      s.alpha = gamma / (delta - s.beta * gamma / h.alpha);
     }
     if (leader) {
       sc->inner_its = k;
@@ -768,58 +819,40 @@ struct Fused32T {
     st1[c] = St4f{rc, sc_, wc, pc};
     return sums(rc, rc * di, wc);
   }
-  DM_HD Red<6> run(int lo, int hi, int t, int nt, const Scal& s) const {
+  DM_HD Pre load(int c) const {
+    Pre p;
     const int n = J.n, w = J.w;
-    const float beta = float(s.beta), alpha = float(s.alpha), um = float(s.um);
-    Red<6> acc = red_identity<6, false>();
-    for (int c0 = lo + t; c0 < hi; c0 += CG_U * nt) {
-      int cc[CG_U];
-      St4f o[CG_U];
-      float di[CG_U], ch[CG_U][WC], g[CG_U][WC];
-      float eo[CG_U];
-      int jj[CG_U][WC];
+    int jj[WC > 0 ? WC : 1];
 #pragma unroll
-      for (int u = 0; u < CG_U; ++u) {
-        cc[u] = (c0 + u * nt < hi) ? c0 + u * nt : c0;
-        o[u] = st0[cc[u]];
-        di[u] = J.dinv32[cc[u]];
-        eo[u] = e[cc[u]];
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) {
-          const bool live = kk < w;
-          const size_t q = size_t(live ? kk : 0) * n + cc[u];
-          const int j = J.nbr[q];
-          const float h = J.chat32[q];
-          jj[u][kk] = (live && j >= 0) ? j : cc[u];
-          ch[u][kk] = live ? h : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < CG_U; ++u)
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) {
-          const St4f nj = st0[jj[u][kk]];
-          g[u][kk] = nj.r - alpha * (nj.w + beta * nj.s);
-        }
-#pragma unroll
-      for (int u = 0; u < CG_U; ++u) {
-        const float uc = o[u].r * di[u] - um;
-        const float pc = uc + beta * o[u].p;
-        const float sc_ = o[u].w + beta * o[u].s;
-        const float rc = o[u].r - alpha * sc_;
-        float wc = rc;
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) wc = wc - ch[u][kk] * g[u][kk];
-        if (c0 + u * nt < hi) {
-          e[cc[u]] = eo[u] + alpha * pc;
-          st1[cc[u]] = St4f{rc, sc_, wc, pc};
-          const Red<6> v = sums(rc, rc * di[u], wc);
-#pragma unroll
-          for (int q = 0; q < 6; ++q) acc.v[q] = acc.v[q] + v.v[q];
-        }
-      }
+    for (int kk = 0; kk < WC; ++kk) {
+      const bool live = kk < w;
+      const size_t q = size_t(live ? kk : 0) * n + c;
+      const int j = J.nbr[q];
+      const float h = J.chat32[q];
+      jj[kk] = (live && j >= 0) ? j : c;
+      p.ch[kk] = live ? h : 0.0f;
     }
-    return acc;
+    p.o = st0[c];
+    p.di = J.dinv32[c];
+    p.e = e[c];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) p.nj[kk] = st0[jj[kk]];
+    return p;
+  }
+  DM_HD void apply(int c, const Pre& p, const Scal& s, Red<6>& acc) const {
+    const float beta = float(s.beta), alpha = float(s.alpha), um = float(s.um);
+    const float uc = p.o.r * p.di - um;
+    const float pc = uc + beta * p.o.p;
+    const float sc_ = p.o.w + beta * p.o.s;
+    const float rc = p.o.r - alpha * sc_;
+    float wc = rc;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) wc = wc - p.ch[kk] * (p.nj[kk].r - alpha * (p.nj[kk].w + beta * p.nj[kk].s));
+    e[c] = p.e + alpha * pc;
+    st1[c] = St4f{rc, sc_, wc, pc};
+    const Red<6> v = sums(rc, rc * p.di, wc);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) acc.v[q] = acc.v[q] + v.v[q];
   }
 };
 using Fused32 = Fused32T<0>;
@@ -896,7 +929,7 @@ struct FcgStart {
 // the fly); partial p.q. The device form (WC > 0) reads WC operator slots branch-free, as FusedT.
 template <int WC>
 struct FcgDirT {
-  static constexpr int kSlots = WC;
+  static constexpr bool kPre = WC > 0;
   EllOp A;
   const double *z, *pold;
   double *pnew, *q;
@@ -905,12 +938,17 @@ struct FcgDirT {
   struct Scal {
     double zm, beta;
   };
-  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s) const {
-    if (sc->done) return false;
-    s.zm = sc->nullspace ? t.v[2] / double(A.n) : 0.0;
+  struct Pre {
+    double cf[WC > 0 ? WC : 1], zj[WC > 0 ? WC : 1], pj[WC > 0 ? WC : 1], z, p, d;
+  };
+  DM_HD Head head() const { return read_head(sc, (k + 1) & 1); }
+  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s) const { return setup(t, leader, s, head()); }
+  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done) return false;
+    s.zm = h.nullspace ? t.v[2] / double(A.n) : 0.0;
     const double zr = t.v[0] - s.zm * t.v[3];
     const double zro = t.v[1] - s.zm * t.v[4];
-    s.beta = k == 0 ? 0.0 : fmax(0.0, (zr - zro) / sc->rz_hist[(k + 1) & 1]);
+    s.beta = k == 0 ? 0.0 : fmax(0.0, (zr - zro) / h.rz);
     if (leader) sc->rz_hist[k & 1] = zr;
     return true;
   }
@@ -932,40 +970,48 @@ struct FcgDirT {
     o.v[0] = pc * qc;
     return o;
   }
-  DM_HD Red<1> run(int lo, int hi, int t, int nt, const Scal& s) const {
+  DM_HD double dir(double zv, double pv, const Scal& s) const {
+    return k == 0 ? zv - s.zm : (zv - s.zm) + s.beta * pv;
+  }
+  DM_HD Pre load(int c) const {
+    Pre o;
     const int n = A.n, w = A.w;
     const bool first = k == 0;
-    Red<1> acc = red_identity<1, false>();
-    for (int c = lo + t; c < hi; c += nt) {
-      int jj[WC > 0 ? WC : 1];
-      double cf[WC > 0 ? WC : 1], pj[WC > 0 ? WC : 1];
+    int jj[WC > 0 ? WC : 1];
 #pragma unroll
-      for (int kk = 0; kk < WC; ++kk) {
-        const bool live = kk < w;
-        const size_t q_ = size_t(live ? kk : 0) * n + c;
-        const int j = A.nbr[q_];
-        const double h = A.coef[q_];
-        jj[kk] = (live && j >= 0) ? j : c;
-        cf[kk] = (live && j >= 0) ? h : 0.0;
-      }
-#pragma unroll
-      for (int kk = 0; kk < WC; ++kk)
-        pj[kk] = first ? z[jj[kk]] - s.zm : (z[jj[kk]] - s.zm) + s.beta * pold[jj[kk]];
-      const double pc = first ? z[c] - s.zm : (z[c] - s.zm) + s.beta * pold[c];
-      double qc = A.diag[c] * pc;
-#pragma unroll
-      for (int kk = 0; kk < WC; ++kk) qc = qc - cf[kk] * pj[kk];
-      pnew[c] = pc;
-      q[c] = qc;
-      acc.v[0] = acc.v[0] + pc * qc;
+    for (int kk = 0; kk < WC; ++kk) {
+      const bool live = kk < w;
+      const size_t q_ = size_t(live ? kk : 0) * n + c;
+      const int j = A.nbr[q_];
+      const double h = A.coef[q_];
+      jj[kk] = (live && j >= 0) ? j : c;
+      o.cf[kk] = (live && j >= 0) ? h : 0.0;
     }
-    return acc;
+    o.z = z[c];
+    o.p = first ? 0.0 : pold[c];
+    o.d = A.diag[c];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) {
+      o.zj[kk] = z[jj[kk]];
+      o.pj[kk] = first ? 0.0 : pold[jj[kk]];
+    }
+    return o;
+  }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<1>& acc) const {
+    const double pc = dir(o.z, o.p, s);
+    double qc = o.d * pc;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) qc = qc - o.cf[kk] * dir(o.zj[kk], o.pj[kk], s);
+    pnew[c] = pc;
+    q[c] = qc;
+    acc.v[0] = acc.v[0] + pc * qc;
   }
 };
 using FcgDir = FcgDirT<0>;
 
 // alpha = (z.r) / (p.q); x += alpha p; r_old = r; r -= alpha q; partial r.r
 struct FcgUpd {
+  static constexpr bool kPre = true;
   double *x, *r, *rold;
   const double *p, *q;
   CgScalars* sc;
@@ -973,20 +1019,22 @@ struct FcgUpd {
   struct Scal {
     double alpha;
   };
-  DM_HD bool setup(const Red<1>& t, bool, Scal& s) const {
-    if (sc->done) return false;
-    s.alpha = sc->rz_hist[k & 1] / t.v[0];
+  struct Pre {
+    double x, p, r, q;
+  };
+  DM_HD Head head() const { return read_head(sc, k & 1); }
+  DM_HD bool setup(const Red<1>& t, bool, Scal& s, const Head& h) const {
+    if (h.done) return false;
+    s.alpha = h.rz / t.v[0];
     return true;
   }
-  DM_HD Red<1> operator()(int c, const Scal& s) const {
-    x[c] = x[c] + s.alpha * p[c];
-    const double rc = r[c];
-    rold[c] = rc;
-    const double rn = rc - s.alpha * q[c];
+  DM_HD Pre load(int c) const { return Pre{x[c], p[c], r[c], q[c]}; }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<1>& acc) const {
+    x[c] = o.x + s.alpha * o.p;
+    rold[c] = o.r;
+    const double rn = o.r - s.alpha * o.q;
     r[c] = rn;
-    Red<1> o;
-    o.v[0] = rn * rn;
-    return o;
+    acc.v[0] = acc.v[0] + rn * rn;
   }
 };
 
@@ -1036,7 +1084,7 @@ struct FcgStart32 {
 // sum r_old = sum r + alpha sum q (no r_old stored, and no cancellation in z.(r - r_old)).
 template <int WC>
 struct FcgDir32T {
-  static constexpr int kSlots = WC;
+  static constexpr bool kPre = WC > 0;
   EllOp32 A;
   const float *z, *pold;
   float* pnew;
@@ -1046,13 +1094,18 @@ struct FcgDir32T {
   struct Scal {
     double zm, beta;
   };
-  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s) const {
-    if (sc->done || sc->inner_done) return false;
-    s.zm = sc->nullspace ? t.v[2] / double(A.n) : 0.0;
+  struct Pre {
+    float cf[WC > 0 ? WC : 1], zj[WC > 0 ? WC : 1], pj[WC > 0 ? WC : 1], z, p, d;
+  };
+  DM_HD Head head() const { return read_head(sc, (k + 1) & 1); }
+  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s) const { return setup(t, leader, s, head()); }
+  DM_HD bool setup(const Red<5>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done || h.inner_done) return false;
+    s.zm = h.nullspace ? t.v[2] / double(A.n) : 0.0;
     const double zr = t.v[0] - s.zm * t.v[3];
-    const double al = sc->alpha32;
+    const double al = h.alpha32;
     const double zro = (t.v[0] + al * t.v[1]) - s.zm * (t.v[3] + al * t.v[4]);
-    s.beta = k == 0 ? 0.0 : fmax(0.0, (zr - zro) / sc->rz_hist[(k + 1) & 1]);
+    s.beta = k == 0 ? 0.0 : fmax(0.0, (zr - zro) / h.rz);
     if (leader) sc->rz_hist[k & 1] = zr;
     return true;
   }
@@ -1079,49 +1132,51 @@ struct FcgDir32T {
   }
   // batched form: all WC slot loads, then all neighbour gathers, branch-free (an empty slot reads
   // the cell itself with a zero coefficient)
-  DM_HD Red<1> run(int lo, int hi, int t, int nt, const Scal& s) const {
+  DM_HD Pre load(int c) const {
+    Pre o;
     const int n = A.n, w = A.w;
-    const float zm = float(s.zm), beta = float(s.beta);
     const bool first = k == 0;
-    Red<1> acc = red_identity<1, false>();
-    for (int c = lo + t; c < hi; c += nt) {
-      int jj[WC > 0 ? WC : 1];
-      float cf[WC > 0 ? WC : 1];
-      float zj[WC > 0 ? WC : 1], pj[WC > 0 ? WC : 1];
-      if (A.opair) {  // 16-bit offsets two to a word, every slot live (EllOff16)
+    int jj[WC > 0 ? WC : 1];
+    if (A.opair) {  // 16-bit offsets two to a word, every slot live (EllOff16)
 #pragma unroll
-        for (int m = 0; m < WC / 2; ++m) {
-          const uint32_t pr = A.opair[size_t(m) * n + c];
-          jj[2 * m] = off16_nbr(c, A.obase[2 * m], pr & 0xffffu);
-          jj[2 * m + 1] = off16_nbr(c, A.obase[2 * m + 1], pr >> 16);
-        }
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) cf[kk] = A.ocoef[size_t(kk) * n + c];
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < WC; ++kk) {
-          const bool live = kk < w;
-          const size_t q_ = size_t(live ? kk : 0) * n + c;
-          const int j = A.nbr[q_];
-          const float h = A.coef[q_];
-          jj[kk] = (live && j >= 0) ? j : c;
-          cf[kk] = (live && j >= 0) ? h : 0.0f;
-        }
+      for (int m = 0; m < WC / 2; ++m) {
+        const uint32_t pr = A.opair[size_t(m) * n + c];
+        jj[2 * m] = off16_nbr(c, A.obase[2 * m], pr & 0xffffu);
+        jj[2 * m + 1] = off16_nbr(c, A.obase[2 * m + 1], pr >> 16);
       }
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) o.cf[kk] = A.ocoef[size_t(kk) * n + c];
+    } else {
 #pragma unroll
       for (int kk = 0; kk < WC; ++kk) {
-        zj[kk] = z[jj[kk]];
-        pj[kk] = first ? 0.0f : pold[jj[kk]];
+        const bool live = kk < w;
+        const size_t q_ = size_t(live ? kk : 0) * n + c;
+        const int j = A.nbr[q_];
+        const float h = A.coef[q_];
+        jj[kk] = (live && j >= 0) ? j : c;
+        o.cf[kk] = (live && j >= 0) ? h : 0.0f;
       }
-      const float pc = dir(z[c], first ? 0.0f : pold[c], zm, beta, first);
-      float qc = A.diag[c] * pc;
-#pragma unroll
-      for (int kk = 0; kk < WC; ++kk) qc = qc - cf[kk] * dir(zj[kk], pj[kk], zm, beta, first);
-      pnew[c] = pc;
-      q[c] = qc;
-      acc.v[0] = acc.v[0] + double(pc) * double(qc);
     }
-    return acc;
+    o.z = z[c];
+    o.p = first ? 0.0f : pold[c];
+    o.d = A.diag[c];
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) {
+      o.zj[kk] = z[jj[kk]];
+      o.pj[kk] = first ? 0.0f : pold[jj[kk]];
+    }
+    return o;
+  }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<1>& acc) const {
+    const float zm = float(s.zm), beta = float(s.beta);
+    const bool first = k == 0;
+    const float pc = dir(o.z, o.p, zm, beta, first);
+    float qc = o.d * pc;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) qc = qc - o.cf[kk] * dir(o.zj[kk], o.pj[kk], zm, beta, first);
+    pnew[c] = pc;
+    q[c] = qc;
+    acc.v[0] = acc.v[0] + double(pc) * double(qc);
   }
 };
 using FcgDir32 = FcgDir32T<0>;
@@ -1129,6 +1184,7 @@ using FcgDir32 = FcgDir32T<0>;
 // alpha = (z.r) / (p.q) (kept for the next direction's beta); e += alpha p; r -= alpha q;
 // partial r.r
 struct FcgUpd32 {
+  static constexpr bool kPre = true;
   float *e, *r;
   const float* p;  // the direction
   const float* q;
@@ -1137,21 +1193,23 @@ struct FcgUpd32 {
   struct Scal {
     double alpha;
   };
-  DM_HD bool setup(const Red<1>& t, bool leader, Scal& s) const {
-    if (sc->done || sc->inner_done) return false;
-    s.alpha = sc->rz_hist[k & 1] / t.v[0];
+  struct Pre {
+    float e, p, r, q;
+  };
+  DM_HD Head head() const { return read_head(sc, k & 1); }
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal& s, const Head& h) const {
+    if (h.done || h.inner_done) return false;
+    s.alpha = h.rz / t.v[0];
     if (leader) sc->alpha32 = s.alpha;
     return true;
   }
-  DM_HD Red<1> operator()(int c, const Scal& s) const {
+  DM_HD Pre load(int c) const { return Pre{e[c], p[c], r[c], q[c]}; }
+  DM_HD void apply(int c, const Pre& o, const Scal& s, Red<1>& acc) const {
     const float a = float(s.alpha);
-    e[c] = e[c] + a * p[c];
-    const float rc = r[c];
-    const float rn = rc - a * q[c];
+    e[c] = o.e + a * o.p;
+    const float rn = o.r - a * o.q;
     r[c] = rn;
-    Red<1> o;
-    o.v[0] = double(rn) * double(rn);
-    return o;
+    acc.v[0] = acc.v[0] + double(rn) * double(rn);
   }
 };
 
@@ -1460,7 +1518,9 @@ class CgT {
       for (;;) {
         for (int i = 0; i < batch; ++i, ++k) {
           xx.tbegin(K_CG_DIR);
-          xx.template pass<4, 1>(n, Dir{A, z_, pold, pnew, q_, sc_, k}, U[(k + 2) % 3], g, D);
+          by_width(A.w, [&](auto wc) {
+            xx.template pass<4, 1>(n, DirT<decltype(wc)::value>{A, z_, pold, pnew, q_, sc_, k}, U[(k + 2) % 3], g, D);
+          });
           xx.tend(K_CG_DIR);
           xx.tbegin(K_CG_UPD);
           xx.template pass<1, 4>(n, Upd{A.diag, pnew, q_, x, r_, z_, sc_, k}, D, g, U[k % 3]);

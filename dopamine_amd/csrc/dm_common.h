@@ -65,16 +65,17 @@ DM_INLINE Red<N> red_identity() {
 
 inline int nblocks(int64_t n, int b = BLOCK) { return int((n + b - 1) / b); }
 
-// A pass functor with a positive static kSlots streams its chunk itself (run(lo, hi, thread,
-// threads, scalars) returns the thread's partials, accumulated in the same cell order as the
-// generic loop); the others are called cell by cell.
+// A pass functor with a static kPre = true splits its work on a cell into load(c) -> Pre, which
+// reads everything that does not depend on the pass's scalars, and apply(c, pre, scalars, sums);
+// its setup() takes the solve's scalars (head()) as an argument. A block then has its first cells'
+// operands and the scalars in flight while it sums the previous pass's partials.
 template <class F, class = void>
-struct PassSlots {
-  static constexpr int value = 0;
+struct PassPre {
+  static constexpr bool value = false;
 };
 template <class F>
-struct PassSlots<F, std::void_t<decltype(F::kSlots)>> {
-  static constexpr int value = F::kSlots;
+struct PassPre<F, std::void_t<decltype(F::kPre)>> {
+  static constexpr bool value = F::kPre;
 };
 
 // ------------------------------------------------------------------ host execution (tests only)
@@ -119,11 +120,16 @@ struct HostExec {
     for (int q = 0; q < in_g; ++q)
       for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
     typename F::Scal sc;
-    if (!f.setup(tot, true, sc)) return;
     Red<NOUT> acc = red_identity<NOUT, false>();
-    if constexpr (PassSlots<F>::value > 0) {  // the batched form the device runs, one thread
-      acc = f.run(0, n, 0, 1, sc);
+    if constexpr (PassPre<F>::value) {
+      if (!f.setup(tot, true, sc, f.head())) return;
+      for (int c = 0; c < n; ++c) f.apply(c, f.load(c), sc, acc);
+      for (int k = 0; k < NOUT; ++k) out_part[k] = acc.v[k];
+      return;
     } else {
+      if (!f.setup(tot, true, sc)) return;
+    }
+    if constexpr (!PassPre<F>::value) {
       for (int c = 0; c < n; ++c) {
         const Red<NOUT> v = f(c, sc);
         for (int k = 0; k < NOUT; ++k) acc.v[k] = acc.v[k] + v.v[k];

@@ -27,15 +27,31 @@ __device__ inline int xcd_block(int nblk) {
   return (b & 7) * per + (b >> 3);
 }
 
+// One step of a wavefront reduction through the DPP lane network: the value of the lane that CTRL
+// names, and what leaves the reduction unchanged (0, or x itself for a maximum) where it names none.
+template <int CTRL, int ROWS, bool MAX>
+__device__ inline double dpp_step(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const int lo = int(uint32_t(u)), hi = int(uint32_t(u >> 32));
+  const int a = __builtin_amdgcn_update_dpp(MAX ? lo : 0, lo, CTRL, ROWS, 0xf, false);
+  const int b = __builtin_amdgcn_update_dpp(MAX ? hi : 0, hi, CTRL, ROWS, 0xf, false);
+  const double o = __builtin_bit_cast(double, uint64_t(uint32_t(a)) | uint64_t(uint32_t(b)) << 32);
+  return MAX ? fmax(x, o) : x + o;
+}
+// The wavefront's total, in lane 63 (row shifts by 1, 2, 4, 8, then row 15 -> rows 1, 3 and row 31
+// -> rows 2, 3): six steps of register moves instead of six trips through LDS (__shfl_down).
 template <int N, bool MAX>
 __device__ inline Red<N> wave_reduce(Red<N> x) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      const double o = __shfl_down(x.v[k], off, 64);
-      x.v[k] = MAX ? fmax(x.v[k], o) : x.v[k] + o;
-    }
+  for (int k = 0; k < N; ++k) {
+    double v = x.v[k];
+    v = dpp_step<0x111, 0xf, MAX>(v);
+    v = dpp_step<0x112, 0xf, MAX>(v);
+    v = dpp_step<0x114, 0xf, MAX>(v);
+    v = dpp_step<0x118, 0xf, MAX>(v);
+    v = dpp_step<0x142, 0xa, MAX>(v);
+    v = dpp_step<0x143, 0xc, MAX>(v);
+    x.v[k] = v;
   }
   return x;
 }
@@ -47,7 +63,7 @@ __device__ inline Red<N> block_reduce(Red<N> x) {
   __shared__ double sh[NT / 64][N];
   x = wave_reduce<N, MAX>(x);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0)
+  if (lane == 63)
 #pragma unroll
     for (int k = 0; k < N; ++k) sh[w][k] = x.v[k];
   __syncthreads();
@@ -130,53 +146,89 @@ constexpr int PGRID_MAX = DM_PGRID_MAX;  // four blocks of four waves per CU
 template <int NIN, int NOUT, class F>
 __global__ void __launch_bounds__(PBLOCK) k_pass(int n, int chunk, F f, const double* in_part, int in_g,
                                                  double* out_part, int tile) {
-  Red<NIN> tot = red_identity<NIN, false>();
-  if constexpr (NIN > 0) {
-    for (int q = threadIdx.x; q < in_g; q += PBLOCK)
-#pragma unroll
-      for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
-    tot = block_reduce<NIN, false, PBLOCK>(tot);
-  }
   const int b = xcd_block(gridDim.x);
-  typename F::Scal sc;
-  if (!f.setup(tot, b == 0 && threadIdx.x == 0, sc)) return;  // uniform across the grid
-  Red<NOUT> acc = red_identity<NOUT, false>();
   const int lo = b * chunk, hi = min(n, lo + chunk);
   const int per = gridDim.x >> 3;
-  if (tile > 0 && per > 0 && b < (per << 3)) {
-    // the XCD's blocks sweep its run of cells together, tile by tile (block j takes tiles j,
-    // j + per, ...), so the neighbours' records are still in that XCD's L2 when they are read
-    const int x0 = (b / per) * per * chunk, x1 = min(n, x0 + per * chunk);
-    for (int t0 = x0 + (b % per) * tile; t0 < x1; t0 += per * tile) {
-      const int t1 = min(x1, t0 + tile);
-      Red<NOUT> v;
-      if constexpr (PassSlots<F>::value > 0) {
-        v = f.run(t0, t1, int(threadIdx.x), PBLOCK, sc);
-      } else {
-        v = red_identity<NOUT, false>();
-        for (int c = t0 + int(threadIdx.x); c < t1; c += PBLOCK) {
-          const Red<NOUT> w = f(c, sc);
+  // the XCD's blocks sweep its run of cells together, tile by tile (block j takes tiles j,
+  // j + per, ...), so the neighbours' records are still in that XCD's L2 when they are read
+  const bool tiled = tile > 0 && per > 0 && b < (per << 3);
+  const int x1 = tiled ? min(n, ((b / per) + 1) * per * chunk) : hi;
+  const int t00 = tiled ? (b / per) * per * chunk + (b % per) * tile : lo;
+  const int span = tiled ? tile : max(chunk, 1), step = tiled ? per * tile : span;
+  if constexpr (PassPre<F>::value) {
+    // On small and medium operators a pass is a chain of dependent loads, not bandwidth: partials,
+    // their sum, scalars, neighbour indices, gathers. Here the first cells' operands, the scalars
+    // and the partials are in flight together: the two-pass CG at 4,096 cells 7.0 + 4.1 -> 5.3 +
+    // 3.4 us, the FP32 update pass at 7.9 million 45.8 -> 31.3 us, the FP64 direction pass at 4.3
+    // million 125 -> 114 us.
+    const auto head = f.head();
+    int c = t00 + int(threadIdx.x);
+    typename F::Pre pre{};
+    if (c < min(x1, t00 + span)) pre = f.load(c);
+    constexpr int PR = (PGRID_MAX + PBLOCK - 1) / PBLOCK;
+    double pv[PR][NIN > 0 ? NIN : 1];
+    if constexpr (NIN > 0) {
 #pragma unroll
-          for (int k = 0; k < NOUT; ++k) v.v[k] = v.v[k] + w.v[k];
-        }
+      for (int r = 0; r < PR; ++r) {
+        const int q = int(threadIdx.x) + r * PBLOCK;
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) pv[r][k] = q < in_g ? in_part[size_t(k) * in_g + q] : 0.0;
       }
-#pragma unroll
-      for (int k = 0; k < NOUT; ++k) acc.v[k] = acc.v[k] + v.v[k];
     }
-  } else if constexpr (PassSlots<F>::value > 0) {
-    acc = f.run(lo, hi, int(threadIdx.x), PBLOCK, sc);
+    Red<NIN> tot = red_identity<NIN, false>();
+    if constexpr (NIN > 0) {
+#pragma unroll
+      for (int r = 0; r < PR; ++r)
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + pv[r][k];
+      for (int q = int(threadIdx.x) + PR * PBLOCK; q < in_g; q += PBLOCK)
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
+      tot = block_reduce<NIN, false, PBLOCK>(tot);
+    }
+    typename F::Scal sc;
+    if (!f.setup(tot, b == 0 && threadIdx.x == 0, sc, head)) return;  // uniform across the grid
+    Red<NOUT> acc = red_identity<NOUT, false>();
+    bool first = true;
+    for (int t0 = t00; t0 < x1; t0 += step) {
+      const int t1 = min(x1, t0 + span);
+      for (c = t0 + int(threadIdx.x); c < t1; c += PBLOCK) {
+        if (!first) pre = f.load(c);
+        first = false;
+        f.apply(c, pre, sc, acc);
+      }
+    }
+    if constexpr (NOUT > 0) {
+      acc = block_reduce<NOUT, false, PBLOCK>(acc);
+      if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < NOUT; ++k) out_part[size_t(k) * gridDim.x + b] = acc.v[k];
+    }
   } else {
-    for (int c = lo + int(threadIdx.x); c < hi; c += PBLOCK) {
-      const Red<NOUT> v = f(c, sc);
+    Red<NIN> tot = red_identity<NIN, false>();
+    if constexpr (NIN > 0) {
+      for (int q = threadIdx.x; q < in_g; q += PBLOCK)
 #pragma unroll
-      for (int k = 0; k < NOUT; ++k) acc.v[k] = acc.v[k] + v.v[k];
+        for (int k = 0; k < NIN; ++k) tot.v[k] = tot.v[k] + in_part[size_t(k) * in_g + q];
+      tot = block_reduce<NIN, false, PBLOCK>(tot);
     }
-  }
-  if constexpr (NOUT > 0) {
-    acc = block_reduce<NOUT, false, PBLOCK>(acc);
-    if (threadIdx.x == 0)
+    typename F::Scal sc;
+    if (!f.setup(tot, b == 0 && threadIdx.x == 0, sc)) return;  // uniform across the grid
+    Red<NOUT> acc = red_identity<NOUT, false>();
+    for (int t0 = t00; t0 < x1; t0 += step) {
+      const int t1 = min(x1, t0 + span);
+      for (int c = t0 + int(threadIdx.x); c < t1; c += PBLOCK) {
+        const Red<NOUT> v = f(c, sc);
 #pragma unroll
-      for (int k = 0; k < NOUT; ++k) out_part[size_t(k) * gridDim.x + b] = acc.v[k];
+        for (int k = 0; k < NOUT; ++k) acc.v[k] = acc.v[k] + v.v[k];
+      }
+    }
+    if constexpr (NOUT > 0) {
+      acc = block_reduce<NOUT, false, PBLOCK>(acc);
+      if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < NOUT; ++k) out_part[size_t(k) * gridDim.x + b] = acc.v[k];
+    }
   }
 }
 
