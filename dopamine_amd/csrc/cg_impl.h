@@ -33,6 +33,13 @@ struct CgScalars {
   double alpha32;                       // FP32 flexible CG: the last update's alpha
 };
 
+// What the host learns of a running solve: written by the device into pinned host memory (device
+// memory for a solve on caller memory), read after the stream has been synchronised.
+struct CgReport {
+  int done, inner_done, its, inner_its;
+  double rr, rr0, target, ttol, atol, resid2;
+};
+
 struct EllOp {
   int n = 0, w = 0;
   const int* nbr = nullptr;      // w*n, -1 = empty slot
@@ -254,6 +261,64 @@ DM_INLINE Head read_head(const CgScalars* s, int at) {
   return Head{s->done, s->inner_done, s->its, s->maxit, s->nullspace, s->ttol, s->inner_tol2, s->rz_hist[at],
               s->gamma_hist[at], s->alpha_hist[at], s->alpha32};
 }
+
+// the solve's scalars from the launch's arguments (an upload would wait for the stream)
+struct SetScalars {
+  CgScalars* sc;
+  CgScalars v;
+  DM_HD void operator()(int) const { *sc = v; }
+};
+
+// One block between batches of iterations: the convergence test that iteration k's first pass is
+// going to make, on the same partials in the same order, and the report the host decides by.
+// rr / rr0 the residual now and at the start (of the sweep), target the one that ends it.
+struct Test {
+  CgScalars* sc;
+  CgReport* rep;
+  int inner, k;
+  using Scal = NoScal;
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal&) const {
+    if (!leader) return false;
+    const double rr = t.v[0];
+    if (!sc->done && !(inner && sc->inner_done)) {
+      if (!inner) {
+        sc->its = k;
+        sc->rr = rr;
+        sc->done = (sqrt(rr) <= sc->ttol) ? 1 : (k >= sc->maxit ? 2 : 0);
+      } else {
+        sc->inner_its = k;
+        if (k > 0 && (rr <= sc->inner_tol2 || sc->its + k >= sc->maxit)) sc->inner_done = 1;
+      }
+    }
+    rep->done = sc->done;
+    rep->inner_done = sc->inner_done;
+    rep->its = sc->its;
+    rep->inner_its = sc->inner_its;
+    rep->rr = rr;
+    const double bn = sc->ttol / fmax(sc->rtol, 1.0e-300);
+    rep->rr0 = inner ? sc->rr : bn * bn;
+    rep->target = inner ? sc->inner_tol2 : sc->ttol * sc->ttol;
+    return false;
+  }
+  DM_HD Red<0> operator()(int, const Scal&) const { return Red<0>{}; }
+};
+
+// the end of a solve: the true residual's sum and what the caller is told
+struct ReportResid {
+  const CgScalars* sc;
+  CgReport* rep;
+  using Scal = NoScal;
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal&) const {
+    if (!leader) return false;
+    rep->done = sc->done;
+    rep->its = sc->its;
+    rep->ttol = sc->ttol;
+    rep->atol = sc->atol;
+    rep->resid2 = t.v[0];
+    return false;
+  }
+  DM_HD Red<0> operator()(int, const Scal&) const { return Red<0>{}; }
+};
 
 // b' = finite(b), x scrubbed; partial: sum b'
 struct SumB {
@@ -1256,20 +1321,20 @@ class CgT {
     q_ = x->template alloc<double>(n);
     sc_ = x->template alloc<CgScalars>(1);
     part_ = x->template alloc<double>(size_t(PARTS) * g_);
-    hpart_.resize(g_);
-    hp_ = hpart_.data();
+    rep_ = x->template alloc_host<CgReport>(1);
   }
   // Bytes of caller memory that init_external carves the work vectors and partials from (a
   // multiple of 256; each piece 256-aligned).
   static size_t external_bytes(int n, int g) {
     const auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    return 6 * al(sizeof(double) * size_t(n)) + al(sizeof(CgScalars)) + al(sizeof(double) * PARTS * size_t(g));
+    return 6 * al(sizeof(double) * size_t(n)) + al(sizeof(CgScalars)) + al(sizeof(CgReport)) +
+           al(sizeof(double) * PARTS * size_t(g));
   }
   // The two-pass Jacobi CG on memory the caller owns: the work vectors and partials are carved
-  // from mem (external_bytes(n, pass_grid(n)) bytes in the execution space), the host copy of the
-  // residual partials goes to host_part (pass_grid(n) doubles). Nothing is allocated, here or in
-  // solve(); destroy() releases nothing. Only the plain Jacobi passes run on such a workspace.
-  void init_external(X* x, int n, void* mem, double* host_part) {
+  // from mem (external_bytes(n, pass_grid(n)) bytes in the execution space). Nothing is allocated,
+  // here or in solve(); destroy() releases nothing. Only the plain Jacobi passes run on such a
+  // workspace.
+  void init_external(X* x, int n, void* mem) {
     x_ = x;
     n_ = n;
     g_ = x->pass_grid(n);
@@ -1287,8 +1352,8 @@ class CgT {
     pb_ = reinterpret_cast<double*>(take(sizeof(double) * size_t(n)));
     q_ = reinterpret_cast<double*>(take(sizeof(double) * size_t(n)));
     sc_ = reinterpret_cast<CgScalars*>(take(sizeof(CgScalars)));
+    rep_ = reinterpret_cast<CgReport*>(take(sizeof(CgReport)));
     part_ = reinterpret_cast<double*>(take(sizeof(double) * PARTS * size_t(g_)));
-    hp_ = host_part;
   }
   // Hestenes-Stiefel two passes per iteration (PETSc KSPCG's recurrence) or the single-reduction
   // variant, one pass per iteration.
@@ -1319,6 +1384,10 @@ class CgT {
       fpart32_ = x_->template alloc<double>(size_t(5) * fpart32_g_);
     }
   }
+  // Which kind of solve comes next (the caller's numbering): iteration counts are predicted from
+  // the previous solve of the same kind.
+  static constexpr int KINDS = 16;
+  void set_kind(int k) { kind_ = k < 0 ? 0 : k % KINDS; }
   // The next solves run the plain Jacobi passes, whatever preconditioner is set (the retry of a
   // failed solve).
   void set_plain(bool on) { plain_ = on; }
@@ -1344,6 +1413,8 @@ class CgT {
                     (void*)z32_, (void*)p32_[0], (void*)p32_[1], (void*)q32_, (void*)fpart32_,
                     (void*)coef32_, (void*)diag32_})
       if (p) x_->release(p);
+    if (rep_) x_->release_host(rep_);
+    rep_ = nullptr;
     r32_ = q32_ = coef32_ = diag32_ = nullptr;
     z32_ = p32_[0] = p32_[1] = nullptr;
     fpart32_ = nullptr;
@@ -1373,12 +1444,12 @@ class CgT {
     double* D = part_ + 3 * size_t(g);   // 1 x g
     double* R = part_ + 4 * size_t(g);   // 1 x g
     double* U[3] = {part_ + 5 * size_t(g), part_ + 9 * size_t(g), part_ + 13 * size_t(g)};  // 4 x g each
-    CgScalars h{};
-    h.rtol = rtol;
-    h.atol = atol;
-    h.maxit = maxit;
-    h.nullspace = nullspace ? 1 : 0;
-    xx.upload(sc_, &h, 1);
+    CgScalars h0{};
+    h0.rtol = rtol;
+    h0.atol = atol;
+    h0.maxit = maxit;
+    h0.nullspace = nullspace ? 1 : 0;
+    xx.for_each(1, SetScalars{sc_, h0});
     if (external_ && (single_ || mixed_ || fcg_ || pc32_))
       throw std::runtime_error("an external CG workspace runs the two-pass Jacobi CG only");
     JacobiScaled J;
@@ -1386,19 +1457,42 @@ class CgT {
     xx.template pass<1, 1>(n, SumB{b, bw_, x}, nullptr, 0, P0);
     xx.template pass<1, 2>(n, Init{A, bw_, r_, x, sc_, atol_dev}, P0, g, P1);
     int k = 0;
-    int batch = std::max(4, std::min(maxit + 1, predict_));
-    if (capture_) batch = std::min(batch, 16);  // residual snapshots along the whole solve
     last_sweeps_ = 0;
     FcgPc* fcg = plain_ ? nullptr : fcg_;
     FcgPc32* pc32 = plain_ ? nullptr : pc32_;
+    int& predict = (fcg ? predict_fcg_ : predict_)[kind_];
+    int* predict_sw = predict_sw_[kind_];
+    const auto residual = [&] {
+      xx.template pass<1, 1>(n, Resid{A, b, x}, nullptr, 0, R);
+      xx.template pass<1, 0>(1, ReportResid{sc_, rep_}, R, g, (double*)nullptr);
+    };
+    // The batches end with the test alone, so a batch of exactly the iterations a solve needs runs
+    // no pass in vain, and the host waits for one report. On small systems the true residual is
+    // taken along, in case the batch was the last.
+    const bool small = n <= (1 << 17);
+    bool have_resid = false;
+    CgReport h{};
+    const auto poll = [&](int inner, int kk, const double* rr) {
+      xx.template pass<1, 0>(1, Test{sc_, rep_, inner, kk}, rr, g, (double*)nullptr);
+      have_resid = small && !inner;
+      if (have_resid) residual();
+      h = fetch();
+    };
+    // iterations left by the convergence so far, at most as many again
+    const auto more = [&](int kk) {
+      if (kk == 0) return 4;
+      const double rate = std::log(h.rr0 / h.rr) / kk;
+      const double left = rate > 0.0 ? std::ceil(std::log(h.rr / h.target) / rate) : double((kk + 7) / 8);
+      const int cap = std::max(8, kk);
+      return left >= 1.0 ? (left < cap ? int(left) : cap) : (left < 1.0 ? 1 : cap);
+    };
     if (fcg) {
       double* RR = U[0];
       const int gt = fcg->out_grid(n);
       xx.template pass<2, 1>(n, FcgStart{r_, ro_, sc_}, P1, g, RR);
       double* pold = pa_;
       double* pnew = pb_;
-      batch = std::max(4, std::min(maxit + 1, predict_fcg_));
-      for (;;) {
+      for (int batch = std::min(maxit + 1, predict);; batch = more(k)) {
         for (int i = 0; i < batch; ++i, ++k) {
           fcg->apply(k, r_, ro_, z_, sc_, RR, g, fpart_);  // times its hidden layer as K_CG_DIR
           xx.tbegin(K_CG_UPD);
@@ -1409,9 +1503,8 @@ class CgT {
           xx.tend(K_CG_UPD);
           std::swap(pold, pnew);
         }
-        xx.download(&h, sc_, 1);
+        poll(0, k, RR);
         if (h.done || k > maxit + 1) break;
-        batch = std::max(2, std::min(16, (h.its + 7) / 8));
       }
     } else if (mixed_ && pc32) {
       // FP64 refinement around FP32 flexible-CG sweeps preconditioned by pc32
@@ -1419,14 +1512,13 @@ class CgT {
       double* RR = U[0];
       const int gt = pc32->out_grid32(n);
       const double* in = P1;
-      int total = 0;
       xx.zero(e32_, size_t(n));
       for (int sweep = 0;; ++sweep) {
         xx.template pass<2, 1>(n, FcgStart32{r_, r32_, x, e32_, sc_, sweep, MAX_SWEEPS, tau_}, in, g, RR);
         int kin = 0;
-        int ibatch = std::max(4, std::min(maxit + 1, predict_sw_[std::min(sweep, MAX_SWEEPS)]));
-        for (;;) {
-          for (int i = 0; i < ibatch; ++i, ++kin) {
+        int& pred = predict_sw[std::min(sweep, MAX_SWEEPS)];
+        for (int batch = std::min(maxit + 1, pred);; batch = more(kin)) {
+          for (int i = 0; i < batch; ++i, ++kin) {
             const float* pold = p32_[kin & 1];
             float* pnew = p32_[(kin + 1) & 1];
             pc32->apply32(kin, r32_, q32_, z32_, 1, sc_, RR, g, fpart32_);
@@ -1440,35 +1532,29 @@ class CgT {
             xx.template pass<1, 1>(n, FcgUpd32{e32_, r32_, pnew, q32_, sc_, kin}, D, g, RR);
             xx.tend(K_CG_UPD);
           }
-          xx.download(&h, sc_, 1);
+          poll(1, kin, RR);
           if (h.done || h.inner_done || kin > maxit + 1) break;
-          ibatch = std::max(2, std::min(16, (h.inner_its + 3) / 4));
         }
-        for (int kc : {int(K_CG_DIR), int(K_CG_UPD), int(K_MG_DOWN), int(K_MG_UP)}) xx.tcommit(kc, h.inner_its);
-        predict_sw_[std::min(sweep, MAX_SWEEPS)] = std::max(1, h.inner_its + 1);
+        for (int kc : {int(K_CG_DIR), int(K_CG_UPD), int(K_MG_DOWN), int(K_MG_UP)})
+          xx.tcommit(kc, h.done ? 0 : h.inner_its);
+        pred = h.done ? 0 : h.inner_its;
         if (h.done) break;
-        total += h.inner_its;
         last_sweeps_ = sweep + 1;
-        h.its = total;
         xx.template pass<1, 2>(n, IrResid{A, bw_, x, e32_, r_, sc_}, nullptr, 0, P1);
         in = P1;
         if (sweep + 1 > MAX_SWEEPS) break;
       }
       xx.for_each(n, IrFold{x, e32_});
-      h.its = total;
     } else if (mixed_) {
       double* F[2] = {U[0], U[0] + 6 * size_t(g)};
       const double* in = P1;
-      int total = 0;
       xx.zero(e32_, size_t(n));
       for (int sweep = 0;; ++sweep) {
         xx.template pass<2, 6>(n, IrStart{J, r_, st32_[0], x, e32_, sc_, sweep, MAX_SWEEPS, tau_}, in, g, F[0]);
         int kin = 0;
-        // sized from the same sweep of the previous solve; later batches a quarter of the
-        // iterations so far (a pass after the stop costs a few microseconds, a host poll more)
-        int ibatch = std::max(8, std::min(maxit + 1, predict_sw_[std::min(sweep, MAX_SWEEPS)]));
-        for (;;) {
-          for (int i = 0; i < ibatch; ++i, ++kin) {
+        int& pred = predict_sw[std::min(sweep, MAX_SWEEPS)];
+        for (int batch = std::min(maxit + 1, pred);; batch = more(kin)) {
+          for (int i = 0; i < batch; ++i, ++kin) {
             const int a = kin & 1, b2 = a ^ 1;
             xx.tbegin(K_CG_DIR);
             by_width(J.w, [&](auto wc) {
@@ -1477,27 +1563,24 @@ class CgT {
             });
             xx.tend(K_CG_DIR);
           }
-          xx.download(&h, sc_, 1);
+          poll(1, kin, F[kin & 1]);
           if (h.done || h.inner_done || kin > maxit + 1) break;
-          ibatch = std::max(8, std::min(64, (h.inner_its + 3) / 4));
         }
-        xx.tcommit(K_CG_DIR, h.inner_its);
-        predict_sw_[std::min(sweep, MAX_SWEEPS)] = std::max(1, h.inner_its + 1);
+        xx.tcommit(K_CG_DIR, h.done ? 0 : h.inner_its);
+        pred = h.done ? 0 : h.inner_its;
         if (h.done) break;
-        total += h.inner_its;
         last_sweeps_ = sweep + 1;
-        h.its = total;
         // IrResid adds the sweep's inner iterations to the device-side count
         xx.template pass<1, 2>(n, IrResid{A, bw_, x, e32_, r_, sc_}, nullptr, 0, P1);
         in = P1;
         if (sweep + 1 > MAX_SWEEPS) break;
       }
       xx.for_each(n, IrFold{x, e32_});  // the last sweep's correction, when no sweep start followed
-      h.its = total;
     } else if (single_) {
       double* F[2] = {U[0], U[0] + 6 * size_t(g)};  // 6 x g each, over the U blocks
       xx.template pass<2, 6>(n, W0{J, r_, st_[0], sc_}, P1, g, F[0]);
-      for (;;) {
+      for (int batch = std::min(maxit + 1, predict);; batch = more(k)) {
+        if (capture_) batch = std::min(batch, 16);  // residual snapshots along the whole solve
         for (int i = 0; i < batch; ++i, ++k) {
           const int a = k & 1, b2 = a ^ 1;
           xx.tbegin(K_CG_DIR);
@@ -1506,16 +1589,16 @@ class CgT {
           });
           xx.tend(K_CG_DIR);
         }
-        xx.download(&h, sc_, 1);
+        poll(0, k, F[k & 1]);
         if (h.done || k > maxit + 1) break;
         if (capture_) capture_->residual(k, &st_[k & 1]->r, 4);
-        batch = std::max(2, std::min(capture_ ? 16 : 32, (h.its + 7) / 8));
       }
     } else {
       xx.template pass<2, 4>(n, Z0{A.diag, r_, z_, sc_}, P1, g, U[2]);
       double* pold = pa_;
       double* pnew = pb_;
-      for (;;) {
+      for (int batch = std::min(maxit + 1, predict);; batch = more(k)) {
+        if (capture_) batch = std::min(batch, 8);
         for (int i = 0; i < batch; ++i, ++k) {
           xx.tbegin(K_CG_DIR);
           by_width(A.w, [&](auto wc) {
@@ -1527,30 +1610,39 @@ class CgT {
           xx.tend(K_CG_UPD);
           std::swap(pold, pnew);
         }
-        xx.download(&h, sc_, 1);
+        poll(0, k, U[(k + 2) % 3]);
         if (h.done || k > maxit + 1) break;
         if (capture_) capture_->residual(k, r_, 1);
-        batch = std::max(2, std::min(capture_ ? 8 : 16, (h.its + 7) / 8));
       }
     }
-    xx.template pass<1, 1>(n, Resid{A, b, x}, nullptr, 0, R);
-    xx.download(hp_, R, size_t(g));
-    xx.download(&h, sc_, 1);
-    double rr = 0.0;
-    for (int q = 0; q < g; ++q) rr = rr + hp_[q];
-    if (!mixed_ || pc32)
+    if (!have_resid) {
+      residual();
+      h = fetch();
+    }
+    if (!mixed_ || !pc32)
       for (int kc : {int(K_CG_DIR), int(K_CG_UPD), int(K_MG_DOWN), int(K_MG_UP)}) xx.tcommit(kc, h.its);
     last_its_ = h.its;
     last_ttol_ = h.ttol;
     last_atol_ = h.atol;
-    (fcg ? predict_fcg_ : predict_) = std::max(2, h.its + 1);
+    if (!mixed_) predict = h.its;
     if (its) *its = h.its;
-    if (resid) *resid = std::sqrt(rr);
+    if (resid) *resid = std::sqrt(h.resid2);
     return h.done == 1 ? 0 : -1;
   }
   static constexpr int MAX_SWEEPS = 40;
 
  private:
+  // the device's report (waits for the stream)
+  CgReport fetch() {
+    CgReport h;
+    if (external_) {
+      x_->download(&h, rep_, 1);
+    } else {
+      x_->sync();
+      h = *rep_;
+    }
+    return h;
+  }
   // Calls fn with the slot count of the batched passes for an operator of width w (0: generic).
   template <class Fn>
   static void by_width(int w, Fn&& fn) {
@@ -1650,16 +1742,15 @@ class CgT {
   double *ro_ = nullptr, *fpart_ = nullptr;
   int fpart_g_ = 0;
   double tau_ = 1e-3;
-  int predict_sw_[MAX_SWEEPS + 1] = {};
+  // iterations of the last solve of each kind (of each sweep, mixed precision)
+  int predict_sw_[KINDS][MAX_SWEEPS + 1] = {}, predict_[KINDS] = {}, predict_fcg_[KINDS] = {}, kind_ = 0;
   int last_sweeps_ = 0;
   double* part_ = nullptr;
   CgScalars* sc_ = nullptr;
-  std::vector<double> hpart_;
-  double* hp_ = nullptr;   // host copy of the residual partials (hpart_ or the caller's array)
+  CgReport* rep_ = nullptr;  // pinned host memory (external: in the caller's memory)
   bool external_ = false;  // work vectors carved from caller memory (init_external)
-  int last_its_ = 0, predict_ = 24;
+  int last_its_ = 0;
   double last_ttol_ = 0.0, last_atol_ = 0.0;
-  int predict_fcg_ = 24;
 };
 
 }  // namespace dm

@@ -91,6 +91,9 @@ struct HostExec {
   }
   void release(void* p) { std::free(p); }
   template <class T>
+  T* alloc_host(size_t n) { return alloc<T>(n); }
+  void release_host(void* p) { std::free(p); }
+  template <class T>
   void upload(T* dst, const T* src, size_t n) { if (n) std::memcpy(dst, src, n * sizeof(T)); }
   template <class T>
   void download(T* dst, const T* src, size_t n) { if (n) std::memcpy(dst, src, n * sizeof(T)); }

@@ -389,6 +389,15 @@ struct DeviceExec {
     return p;
   }
   void release(void* p) { if (p) (void)hipFree(p); }
+  // pinned host memory that kernels write
+  template <class T>
+  T* alloc_host(size_t n) {
+    void* p = nullptr;
+    DM_CHECK(hipHostMalloc(&p, (n ? n : 1) * sizeof(T), hipHostMallocDefault));
+    std::memset(p, 0, (n ? n : 1) * sizeof(T));
+    return static_cast<T*>(p);
+  }
+  void release_host(void* p) { if (p) (void)hipHostFree(p); }
   template <class T>
   void upload(T* dst, const T* src, size_t n) {
     if (n) DM_CHECK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, stream));

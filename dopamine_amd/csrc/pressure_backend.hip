@@ -199,7 +199,7 @@ constexpr size_t NOALLOC_DIAG_BYTES = noalloc_al(sizeof(double) * size_t(NOALLOC
 constexpr size_t NOALLOC_OP_BYTES = NOALLOC_NBR_BYTES + NOALLOC_COEF_BYTES + NOALLOC_DIAG_BYTES;
 // the CG's work vectors and partials for the largest operator (the pass grid never exceeds PGRID_MAX)
 constexpr size_t NOALLOC_CG_BYTES = 6 * noalloc_al(sizeof(double) * size_t(NOALLOC_MAX_CELLS)) +
-                                    noalloc_al(sizeof(dm::CgScalars)) +
+                                    noalloc_al(sizeof(dm::CgScalars)) + noalloc_al(sizeof(dm::CgReport)) +
                                     noalloc_al(sizeof(double) * 17 * size_t(dm::PGRID_MAX));
 constexpr size_t NOALLOC_BYTES = NOALLOC_OP_BYTES + NOALLOC_CG_BYTES;
 
@@ -210,7 +210,6 @@ int h_cnt[NOALLOC_MAX_CELLS];
 int h_nbr[NOALLOC_MAX_WIDTH * NOALLOC_MAX_CELLS];
 double h_coef[NOALLOC_MAX_WIDTH * NOALLOC_MAX_CELLS];
 double h_diag[NOALLOC_MAX_CELLS];
-double h_part[dm::PGRID_MAX];
 char g_noalloc_error[256] = "";
 
 // Device address of this GPU's scratch array (looked up on the first call on each device).
@@ -311,7 +310,7 @@ int fvm_petsc_solve_pressure_noalloc(int n_cells_local, int n_cells_global, int 
     dm::CgT<dm::DeviceExec> cg;
     if (dm::CgT<dm::DeviceExec>::external_bytes(n, ex.pass_grid(n)) > NOALLOC_CG_BYTES)
       return fail(-63, "scratch too small for the CG workspace");
-    cg.init_external(&ex, n, base + NOALLOC_OP_BYTES, h_part);
+    cg.init_external(&ex, n, base + NOALLOC_OP_BYTES);
     dm::EllOp A;
     A.n = n;
     A.w = w;

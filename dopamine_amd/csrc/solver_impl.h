@@ -1370,7 +1370,11 @@ class SolverT {
     x.download(&h, sc, 1);
     return h.pj[i];
   }
+  // kinds of solves for the CG's iteration forecasts: the stage's non-orthogonal correctors, the
+  // initial projections, the exact projection's preconditioner
+  static constexpr int KIND_ONCE = 14, KIND_PRECOND = 15;
   void pj_precond() {
+    cg.set_kind(KIND_PRECOND);
     x.zero(pj_z, nc);
     int its = 0;
     double res = 0.0;
@@ -1444,6 +1448,7 @@ class SolverT {
     int rc = 0;
     if (prm.p_max_iter > 0) {
       atol_for(dt);
+      cg.set_kind(KIND_ONCE);
       rc = pressure_solve(true, &sc->atol, 0.0);
     }
     anchor_pressure();
@@ -1606,6 +1611,7 @@ class SolverT {
         for (int jno = 1; jno <= nmax; ++jno) {
           face_fluxes_and_rhs(gdt, jno > 1);
           if (jno == 1) x.zero(P, nc);
+          cg.set_kind(4 * k + std::min(jno, 4) - 1);
           if (pressure_solve(false, &sc->atol, 0.0) != 0) rc = -2;
           bc_pressure(1, skip_grad_p ? nullptr : gp, 0.0, nullptr);
           bc_pressure(2, nullptr, 0.0, nullptr);
