@@ -358,6 +358,8 @@ struct AmgCfg {
   // product instead of three kernels (2,457 cells on the channel: 24 MB in 5.9 us, where the
   // three took 3 x 3-4 us; the line lies where the matrix takes as long to read as the kernels).
   int dense_max = 2816;
+  // Level 0 takes the row table where it has at least this many cells per distinct row (0: never).
+  int row_share = 16;
   int max_levels = 16;
 };
 
@@ -439,8 +441,12 @@ struct AmgLevelDev {
   const AmgCoef *cs = nullptr, *cr = nullptr;    // level 0: scaled couplings [slot][cell]
   // level 0, when its neighbour offsets fit 16 bits (EllOff16): each slot's coupling and offset
   // in one word (binary16 coupling in the low half, offset - obase[slot] in the high half)
-  const uint32_t *hs = nullptr, *hr = nullptr;
+  const uint32_t* hr = nullptr;
   int obase[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  // or, when the operator has a row table (RowTable): the row of each cell and the post-smoothing's
+  // records (offsets, cr, 1 / diag)
+  const uint16_t* rid = nullptr;
+  const void* rup = nullptr;
   const float* dinv = nullptr;
   AmgMat<AmgCoef> S;                             // coarse levels: the couplings cs
   AmgMat<float> R, Q;                            // R to the next level; coarse levels: Q = R^T
@@ -794,14 +800,24 @@ struct Up0 {
   DM_HD Pre load(int c) const {
     Pre o;
     int jj[WC > 0 ? WC : 1];
-    if (L.hr)
-      slots0p<WC>(L, L.hr, c, jj, o.h);
-    else
-      slots0<WC>(L, L.cr, c, jj, o.h);
     o.x = L.x[c];
-    o.di = L.dinv[c];
     o.r = r[c];
     o.ro = rold[c];
+    if (L.rid) {
+      const RowRec<(WC > 0 ? WC : 4)> row = row_rec<(WC > 0 ? WC : 4)>(L.rup, L.rid[c]);
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) {
+        jj[kk] = c + row.off[kk];
+        o.h[kk] = row.v[kk];
+      }
+      o.di = row.d;
+    } else {
+      if (L.hr)
+        slots0p<WC>(L, L.hr, c, jj, o.h);
+      else
+        slots0<WC>(L, L.cr, c, jj, o.h);
+      o.di = L.dinv[c];
+    }
 #pragma unroll
     for (int kk = 0; kk < WC; ++kk) o.xj[kk] = L.x[jj[kk]];
     return o;
@@ -864,7 +880,7 @@ class AmgPc : public FcgPc, public FcgPc32 {
       L.dinv = up(di.back());
       const auto scaled = scaled_of(lev);
       if (lev == 0) {
-        build_level0(L, cur, nbr_dev, scaled);
+        build_level0(L, cur, nbr_dev, di.back().data(), scaled);
       } else {  // the non-empty entries, packed rows
         AmgCsr S;
         S.ptr.assign(size_t(cur.n) + 1, 0);
@@ -962,6 +978,11 @@ class AmgPc : public FcgPc, public FcgPc32 {
   bool singular() const { return singular_; }
   double alpha() const { return alpha_; }
   bool aggressive() const { return aggressive_; }
+  // The operator's row table for the direction pass (its rows' coefficients and diagonals), or none.
+  void share_rows(EllOp& A) const {
+    A.rid = levels_[0].rid;
+    A.rrec = rdir_;
+  }
   const AmgCfg& cfg() const { return cfg_; }
 
   // ---- FcgPc (FP64 flexible CG)
@@ -986,7 +1007,7 @@ class AmgPc : public FcgPc, public FcgPc32 {
  private:
   // level 0: the solver's neighbour array with the scaled couplings, and their compact form
   template <class Scaled>
-  void build_level0(AmgLevelDev& L, const AmgOp& cur, const int* nbr_dev, Scaled&& scaled) {
+  void build_level0(AmgLevelDev& L, const AmgOp& cur, const int* nbr_dev, const float* dinv, Scaled&& scaled) {
     L.w = cur.w;
     L.nbr = nbr_dev;
     const size_t m = size_t(std::max(1, cur.w)) * cur.n;
@@ -1002,17 +1023,31 @@ class AmgPc : public FcgPc, public FcgPc32 {
     const std::vector<AmgCoef> hcs = to_coef(cs), hcr = to_coef(cr);
     L.cs = up(hcs);
     L.cr = up(hcr);
+    if (!off16_enabled()) return;
+    RowTable t;
+    const auto rounded = [&](int, size_t q, float* a, float* b) {
+      *a = coef_f(hcs[q]);
+      *b = coef_f(hcr[q]);
+    };
+    if (row_table(cur.nbr.data(), cur.coef.data(), cur.diag.data(), dinv, cur.n, cur.w, cfg_.row_share, rounded, t)) {
+      L.rid = up(t.id);
+      with_width(t.W, [&](auto wc) {
+        constexpr int W = decltype(wc)::value;
+        if constexpr (W > 0) {
+          L.rup = up(row_recs<W>(t, t.cr, t.dinv));
+          rdir_ = up(row_recs<W>(t, t.coef, t.diag));
+        }
+      });
+      return;
+    }
     EllOff16 o16;
-    if (off16_enabled() && ell_off16(cur.nbr.data(), cur.n, cur.w, o16)) {
-      std::vector<uint32_t> ws(size_t(o16.W) * cur.n), wr(ws.size());
-      for (size_t q = 0; q < ws.size(); ++q) {
+    if (ell_off16(cur.nbr.data(), cur.n, cur.w, o16)) {
+      std::vector<uint32_t> wr(size_t(o16.W) * cur.n);
+      for (size_t q = 0; q < wr.size(); ++q) {
         const int s = o16.src[q];
         const size_t q0 = size_t(s) * cur.n + q % size_t(cur.n);
-        const uint32_t hi = uint32_t(uint16_t(o16.d[q])) << 16;
-        ws[q] = hi | (s < 0 ? 0u : uint32_t(hcs[q0]));
-        wr[q] = hi | (s < 0 ? 0u : uint32_t(hcr[q0]));
+        wr[q] = uint32_t(uint16_t(o16.d[q])) << 16 | (s < 0 ? 0u : uint32_t(hcr[q0]));
       }
-      L.hs = up(ws);
       L.hr = up(wr);
       for (int k = 0; k < 8; ++k) L.obase[k] = o16.base[k];
     }
@@ -1092,6 +1127,7 @@ class AmgPc : public FcgPc, public FcgPc32 {
   std::vector<int> sizes_;
   std::vector<int64_t> nnz_, stored_;
   std::vector<void*> owned_;
+  const void* rdir_ = nullptr;  // the direction pass's records of the row table
   float* dense_ = nullptr;  // the bottom's matrix, rows padded to lda_
   int lda_ = 0, bottom_ = 1;
   double alpha_ = 1.5;

@@ -16,7 +16,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
+#include <cstring>
 #include <stdexcept>
 #include <type_traits>
 #include <vector>
@@ -50,6 +52,9 @@ struct EllOp {
   const uint32_t* opair = nullptr;
   const float* ocoef = nullptr;
   int obase[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  // or its row table (see RowTable): the row of each cell and the rows' records
+  const uint16_t* rid = nullptr;
+  const void* rrec = nullptr;
 };
 
 // Neighbour offsets of an ELL operator in 16 bits, for the batched passes that stream the whole
@@ -163,6 +168,143 @@ inline bool off16_enabled() {
   return !(e && e[0] == '0');
 }
 
+// One row of an operator as the batched FP32 passes read it: its neighbours' offsets j - c, a value
+// per slot and one of the diagonal (empty slots: offset 0, value 0).
+template <int W>
+struct alignas(16) RowRec {
+  int off[W];
+  float v[W];
+  float d;
+  float pad[(4 - (2 * W + 1) % 4) % 4];
+};
+
+// Row table of an operator: most cells of a box mesh (uniform or stretched, with walls, periodic
+// sides or cells cut out) share their row with many others, since an FP32 coefficient absorbs the
+// rounding noise of the geometry. Each distinct row is stored once and a cell keeps a 16-bit
+// number of its row: 2 bytes where the lists hold 36 (direction pass) and 24 (smoothing). The
+// values and the slots are the lists' own, so a pass adds the same terms in the same order. Built
+// when the rows number at most 65,536 and there are at least `share` cells per distinct row on
+// average (jittered meshes have a row per cell and keep their lists).
+struct RowTable {
+  int W = 0, rows = 0;
+  std::vector<uint16_t> id;             // row of each cell
+  std::vector<int> off;                 // [row][W]
+  std::vector<float> coef, cs, cr;      // [row][W]: coefficients, binary16-rounded couplings
+  std::vector<float> diag, dinv;        // [row]
+};
+// scaled(c, q, &cs, &cr) gives the rounded couplings of entry q of cell c (zero where left out),
+// dinv the smoother's diagonal inverses
+template <class Scaled>
+inline bool row_table(const int* nbr, const double* coef, const double* diag, const float* dinv, int n, int w, int share,
+                      Scaled&& scaled, RowTable& o) {
+  const int W = w <= 4 ? 4 : w <= 6 ? 6 : w <= 8 ? 8 : 0;
+  if (W == 0 || n <= 0 || share <= 0) return false;
+  const size_t most = std::min<size_t>(65536, size_t(n) / size_t(share));
+  const int K = 4 * W + 2;  // words of a row's key: offsets, coefficients, couplings, diagonals
+  o.W = W;
+  o.id.assign(n, 0);
+  std::vector<uint32_t> keys;  // of the distinct rows
+  std::vector<int> slot(1 << 18, -1);  // open addressing over the distinct rows' hashes
+  const size_t mask = slot.size() - 1;
+  std::vector<uint32_t> key(K);
+  const auto bits = [](float f) {
+    uint32_t u;
+    std::memcpy(&u, &f, 4);
+    return u;
+  };
+  size_t rows = 0;
+  for (int c = 0; c < n; ++c) {
+    std::fill(key.begin(), key.end(), 0u);
+    for (int k = 0; k < w; ++k) {
+      const size_t q = size_t(k) * n + c;
+      if (nbr[q] < 0) continue;
+      float s = 0.0f, r = 0.0f;
+      scaled(c, q, &s, &r);
+      key[k] = uint32_t(nbr[q] - c);
+      key[W + k] = bits(float(coef[q]));
+      key[2 * W + k] = bits(s);
+      key[3 * W + k] = bits(r);
+    }
+    key[4 * W] = bits(float(diag[c]));
+    key[4 * W + 1] = bits(dinv[c]);
+    uint64_t h = 1469598103934665603ull;
+    for (uint32_t u : key) h = (h ^ u) * 1099511628211ull;
+    size_t at = size_t(h ^ (h >> 29)) & mask;
+    for (;; at = (at + 1) & mask) {
+      if (slot[at] < 0) {
+        if (rows >= most) return false;
+        slot[at] = int(rows++);
+        keys.insert(keys.end(), key.begin(), key.end());
+        break;
+      }
+      if (std::equal(key.begin(), key.end(), keys.begin() + size_t(slot[at]) * K)) break;
+    }
+    o.id[c] = uint16_t(slot[at]);
+  }
+  o.rows = int(rows);
+  const auto val = [](uint32_t u) {
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+  };
+  for (size_t r = 0; r < rows; ++r) {
+    const uint32_t* q = &keys[r * K];
+    for (int k = 0; k < W; ++k) {
+      o.off.push_back(int(q[k]));
+      o.coef.push_back(val(q[W + k]));
+      o.cs.push_back(val(q[2 * W + k]));
+      o.cr.push_back(val(q[3 * W + k]));
+    }
+    o.diag.push_back(val(q[4 * W]));
+    o.dinv.push_back(val(q[4 * W + 1]));
+  }
+  return true;
+}
+// one pass's records of a row table: values v per slot and d per row
+template <int W>
+inline std::vector<RowRec<W>> row_recs(const RowTable& t, const std::vector<float>& v, const std::vector<float>& d) {
+  std::vector<RowRec<W>> o(size_t(t.rows));
+  for (int r = 0; r < t.rows; ++r) {
+    for (int k = 0; k < W; ++k) {
+      o[r].off[k] = t.off[size_t(r) * W + k];
+      o[r].v[k] = v[size_t(r) * W + k];
+    }
+    o[r].d = d[r];
+  }
+  return o;
+}
+// Record `id` of a pass's table. Neighbouring cells mostly share their row: where all of a
+// wavefront's lanes do, it comes through the scalar cache into scalar registers; elsewhere each
+// lane reads its own (L1 / L2).
+template <int W>
+DM_INLINE RowRec<W> row_rec(const void* table, int id) {
+  const RowRec<W>* t = static_cast<const RowRec<W>*>(table);
+#if defined(__HIP_DEVICE_COMPILE__)
+  RowRec<W> o;
+  const int u = __builtin_amdgcn_readfirstlane(id);
+  if (__builtin_amdgcn_ballot_w64(id != u) == 0) {
+    const auto* p = (const __attribute__((address_space(4))) RowRec<W>*)(uintptr_t)(t + u);
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      o.off[k] = p->off[k];
+      o.v[k] = p->v[k];
+    }
+    o.d = p->d;
+    return o;
+  }
+  const RowRec<W>* p = t + id;
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    o.off[k] = p->off[k];
+    o.v[k] = p->v[k];
+  }
+  o.d = p->d;
+  return o;
+#else
+  return t[id];
+#endif
+}
+
 // Packed per-cell state of the single-reduction recurrence: one 32-byte (16-byte in FP32) load
 // fetches everything a neighbour contributes.
 struct alignas(32) St4 {
@@ -241,6 +383,8 @@ struct EllOp32 {
   const uint32_t* opair = nullptr;  // as EllOp: the compact copy, or null
   const float* ocoef = nullptr;
   int obase[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  const uint16_t* rid = nullptr;  // as EllOp: the row table, or null
+  const void* rrec = nullptr;
 };
 
 // Chained passes of one solve. Each reads the totals of the previous pass's partials (identical
@@ -1043,18 +1187,29 @@ struct FcgDirT {
     const int n = A.n, w = A.w;
     const bool first = k == 0;
     int jj[WC > 0 ? WC : 1];
-#pragma unroll
-    for (int kk = 0; kk < WC; ++kk) {
-      const bool live = kk < w;
-      const size_t q_ = size_t(live ? kk : 0) * n + c;
-      const int j = A.nbr[q_];
-      const double h = A.coef[q_];
-      jj[kk] = (live && j >= 0) ? j : c;
-      o.cf[kk] = (live && j >= 0) ? h : 0.0;
-    }
     o.z = z[c];
     o.p = first ? 0.0 : pold[c];
     o.d = A.diag[c];
+    if (A.rid) {  // the neighbours from the row table, the FP64 coefficients from the lists (0 if empty)
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) {
+        const double h = A.coef[size_t(kk < w ? kk : 0) * n + c];
+        o.cf[kk] = kk < w ? h : 0.0;
+      }
+      const RowRec<(WC > 0 ? WC : 4)> r = row_rec<(WC > 0 ? WC : 4)>(A.rrec, A.rid[c]);
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) jj[kk] = c + r.off[kk];
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) {
+        const bool live = kk < w;
+        const size_t q_ = size_t(live ? kk : 0) * n + c;
+        const int j = A.nbr[q_];
+        const double h = A.coef[q_];
+        jj[kk] = (live && j >= 0) ? j : c;
+        o.cf[kk] = (live && j >= 0) ? h : 0.0;
+      }
+    }
 #pragma unroll
     for (int kk = 0; kk < WC; ++kk) {
       o.zj[kk] = z[jj[kk]];
@@ -1202,7 +1357,17 @@ struct FcgDir32T {
     const int n = A.n, w = A.w;
     const bool first = k == 0;
     int jj[WC > 0 ? WC : 1];
-    if (A.opair) {  // 16-bit offsets two to a word, every slot live (EllOff16)
+    o.z = z[c];
+    o.p = first ? 0.0f : pold[c];
+    if (A.rid) {
+      const RowRec<(WC > 0 ? WC : 4)> r = row_rec<(WC > 0 ? WC : 4)>(A.rrec, A.rid[c]);
+#pragma unroll
+      for (int kk = 0; kk < WC; ++kk) {
+        jj[kk] = c + r.off[kk];
+        o.cf[kk] = r.v[kk];
+      }
+      o.d = r.d;
+    } else if (A.opair) {  // 16-bit offsets two to a word, every slot live (EllOff16)
 #pragma unroll
       for (int m = 0; m < WC / 2; ++m) {
         const uint32_t pr = A.opair[size_t(m) * n + c];
@@ -1211,6 +1376,7 @@ struct FcgDir32T {
       }
 #pragma unroll
       for (int kk = 0; kk < WC; ++kk) o.cf[kk] = A.ocoef[size_t(kk) * n + c];
+      o.d = A.diag[c];
     } else {
 #pragma unroll
       for (int kk = 0; kk < WC; ++kk) {
@@ -1221,10 +1387,8 @@ struct FcgDir32T {
         jj[kk] = (live && j >= 0) ? j : c;
         o.cf[kk] = (live && j >= 0) ? h : 0.0f;
       }
+      o.d = A.diag[c];
     }
-    o.z = z[c];
-    o.p = first ? 0.0f : pold[c];
-    o.d = A.diag[c];
 #pragma unroll
     for (int kk = 0; kk < WC; ++kk) {
       o.zj[kk] = z[jj[kk]];
@@ -1706,6 +1870,8 @@ class CgT {
     o.opair = A.opair;
     o.ocoef = A.ocoef;
     for (int k = 0; k < 8; ++k) o.obase[k] = A.obase[k];
+    o.rid = A.rid;
+    o.rrec = A.rrec;
     return o;
   }
   float *coef32_ = nullptr, *diag32_ = nullptr;

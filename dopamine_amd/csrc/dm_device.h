@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(PBLOCK) k_pass(int n, int chunk, F f, const do
     const auto head = f.head();
     int c = t00 + int(threadIdx.x);
     typename F::Pre pre{};
-    if (c < min(x1, t00 + span)) pre = f.load(c);
+    if (c < x1) pre = f.load(c);
     constexpr int PR = (PGRID_MAX + PBLOCK - 1) / PBLOCK;
     double pv[PR][NIN > 0 ? NIN : 1];
     if constexpr (NIN > 0) {
@@ -189,14 +189,13 @@ __global__ void __launch_bounds__(PBLOCK) k_pass(int n, int chunk, F f, const do
     typename F::Scal sc;
     if (!f.setup(tot, b == 0 && threadIdx.x == 0, sc, head)) return;  // uniform across the grid
     Red<NOUT> acc = red_identity<NOUT, false>();
-    bool first = true;
-    for (int t0 = t00; t0 < x1; t0 += step) {
-      const int t1 = min(x1, t0 + span);
-      for (c = t0 + int(threadIdx.x); c < t1; c += PBLOCK) {
-        if (!first) pre = f.load(c);
-        first = false;
-        f.apply(c, pre, sc, acc);
-      }
+    // a thread's cells: one per tile, or every PBLOCK-th of the block's run
+    const int stride = tiled ? step : PBLOCK;
+    for (bool more = c < x1; more;) {
+      f.apply(c, pre, sc, acc);
+      c += stride;
+      more = c < x1;
+      if (more) pre = f.load(c);
     }
     if constexpr (NOUT > 0) {
       acc = block_reduce<NOUT, false, PBLOCK>(acc);
@@ -293,13 +292,13 @@ struct DeviceExec {
   int part_blocks = 0;
   KernelTimer* kt = nullptr;
   int open_ = -1;            // class of the launch being timed
-  // chained passes: each XCD's blocks sweep its cells together in tiles of this many (k_pass);
-  // 0: one contiguous chunk per block. DOPAMINE_PASS_TILE overrides (for tuning).
-  int pass_tile = 256;
+  // chained passes: each XCD's blocks sweep its cells together in tiles of a block's threads
+  // (k_pass); 0: one contiguous chunk per block (DOPAMINE_PASS_TILE=0, for tuning).
+  int pass_tile = PBLOCK;
 
   void init(int max_n) {
     DM_CHECK(hipStreamCreate(&stream));  // default priority
-    if (const char* e = std::getenv("DOPAMINE_PASS_TILE")) pass_tile = std::max(0, std::atoi(e)) / 64 * 64;
+    if (const char* e = std::getenv("DOPAMINE_PASS_TILE")) pass_tile = std::atoi(e) > 0 ? PBLOCK : 0;
     part_blocks = nblocks(max_n > 0 ? max_n : 1);
     DM_CHECK(hipMalloc(&part, sizeof(double) * 8 * size_t(part_blocks)));
     kt = new KernelTimer();

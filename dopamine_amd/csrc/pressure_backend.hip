@@ -128,16 +128,6 @@ int build_ctx(int n, int n_global, int n_faces, const int* l2g, const int* owner
     ctx->A32.diag = ctx->diag32;
     ctx->cg.set_mixed(ctx->A32, 1.0e-4);
     ctx->mixed = true;
-    std::vector<uint32_t> pr;
-    std::vector<float> oc;
-    if (dm::off16_enabled() && dm::ell_pack32(nbr.data(), cf.data(), n, w, pr, oc, ctx->A.obase)) {
-      ctx->opair = ctx->x.alloc<uint32_t>(pr.size());
-      ctx->ocoef = ctx->x.alloc<float>(oc.size());
-      ctx->x.upload(ctx->opair, pr.data(), pr.size());
-      ctx->x.upload(ctx->ocoef, oc.data(), oc.size());
-      ctx->A.opair = ctx->opair;
-      ctx->A.ocoef = ctx->ocoef;
-    }
   }
   if (multigrid_selector(g_solver)) {
     dm::AmgOp op;
@@ -148,9 +138,20 @@ int build_ctx(int n, int n_global, int n_faces, const int* l2g, const int* owner
     op.diag = dg;
     ctx->amg.reset(new dm::AmgPc<dm::DeviceExec>());
     ctx->amg->build(&ctx->x, op, ctx->nbr, dm::AmgCfg{});
-    if (ctx->mixed)
+    ctx->amg->share_rows(ctx->A);
+    if (ctx->mixed) {
       ctx->cg.set_pc32(ctx->amg.get());
-    else
+      std::vector<uint32_t> pr;
+      std::vector<float> oc;
+      if (!ctx->A.rid && dm::off16_enabled() && dm::ell_pack32(nbr.data(), cf.data(), n, w, pr, oc, ctx->A.obase)) {
+        ctx->opair = ctx->x.alloc<uint32_t>(pr.size());
+        ctx->ocoef = ctx->x.alloc<float>(oc.size());
+        ctx->x.upload(ctx->opair, pr.data(), pr.size());
+        ctx->x.upload(ctx->ocoef, oc.data(), oc.size());
+        ctx->A.opair = ctx->opair;
+        ctx->A.ocoef = ctx->ocoef;
+      }
+    } else
       ctx->cg.set_fcg(ctx->amg.get());
   }
   if (g_solver == "fcg-learned") {

@@ -241,7 +241,8 @@ class SolverT {
   // relative residual reduction of one FP32 sweep (DOPAMINE_MIXED_TAU overrides, for tuning)
   // Multigrid set-up: AmgCfg's defaults; DOPAMINE_AMG_THETA / _THETA0 / _ALPHA / _COARSE override
   // the strength thresholds (all levels / the first), the coarse-correction scaling and the
-  // densely solved size; _DENSE the size up to which levels are folded into it.
+  // densely solved size; _DENSE the size up to which levels are folded into it, _ROW_SHARE the
+  // cells per distinct row from which the row table is used.
   static AmgCfg amg_cfg() {
     AmgCfg c;
     if (const char* e = std::getenv("DOPAMINE_AMG_THETA")) c.theta = std::atof(e);
@@ -251,6 +252,7 @@ class SolverT {
     if (const char* e = std::getenv("DOPAMINE_AMG_OMEGA")) c.omega = std::atof(e);
     if (const char* e = std::getenv("DOPAMINE_AMG_COARSE")) c.coarse_max = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("DOPAMINE_AMG_DENSE")) c.dense_max = std::atoi(e);
+    if (const char* e = std::getenv("DOPAMINE_AMG_ROW_SHARE")) c.row_share = std::atoi(e);
     return c;
   }
   static double mixed_tau() {
@@ -693,12 +695,6 @@ class SolverT {
       A32.nbr = A.nbr;
       A32.coef = up(c32);
       A32.diag = up(d32);
-      std::vector<uint32_t> pr;  // the compact copy the batched FP32 direction pass streams
-      std::vector<float> oc;
-      if (off16_enabled() && ell_pack32(anbr.data(), acoef.data(), nc, wP, pr, oc, A.obase)) {
-        A.opair = up(pr);
-        A.ocoef = up(oc);
-      }
     }
     if (n_dir) {
       dir_rows = up(dir_rows_h);
@@ -845,9 +841,16 @@ class SolverT {
       op.diag = diag;
       amg.reset(new AmgPc<X>());
       amg->build(&x, op, A.nbr, amg_cfg());
-      if (p.precision == 1)
+      amg->share_rows(A);
+      if (p.precision == 1) {
         cg.set_pc32(amg.get());
-      else
+        std::vector<uint32_t> pr;  // else the compact copy the batched FP32 direction pass streams
+        std::vector<float> oc;
+        if (!A.rid && off16_enabled() && ell_pack32(anbr.data(), acoef.data(), nc, wP, pr, oc, A.obase)) {
+          A.opair = up(pr);
+          A.ocoef = up(oc);
+        }
+      } else
         cg.set_fcg(amg.get());
     }
     apply_all_bc();

@@ -141,10 +141,40 @@ int hc_ell_off16(int n, int w, const int* nbr, int* base, int16_t* d, int* src) 
 }
 // Size up to which levels are folded into the cycle's dense bottom (AmgCfg::dense_max; negative:
 // the product's).
-static int g_dense_max = -1;
+static int g_dense_max = -1, g_row_share = -1;
 void hc_amg_dense_max(int m) { g_dense_max = m; }
+// Cells per distinct row from which level 0 takes the row table (AmgCfg::row_share; 0 never,
+// negative the product's).
+void hc_amg_row_share(int m) { g_row_share = m; }
 static void layout(dm::AmgCfg& c) {
   if (g_dense_max >= 0) c.dense_max = g_dense_max;
+  if (g_row_share >= 0) c.row_share = g_row_share;
+}
+// The row table of an ELL operator with unit couplings: the number of distinct rows (0: none) and,
+// through the pass's record reader, every cell's neighbours and coefficients (W * n, empty slots
+// the cell itself and 0); W in *width.
+int hc_row_table(int n, int w, const int* nbr, const double* coef, const double* diag, int share, int* width, int* jout,
+                 float* vout, float* dout) {
+  std::vector<float> di(n, 1.0f);
+  dm::RowTable t;
+  if (!dm::row_table(nbr, coef, diag, di.data(), n, w, share, [](int, size_t, float* a, float* b) { *a = *b = 1.0f; }, t))
+    return 0;
+  *width = t.W;
+  dm::with_width(t.W, [&](auto wc) {
+    constexpr int W = decltype(wc)::value;
+    if constexpr (W > 0) {
+      const auto rec = dm::row_recs<W>(t, t.coef, t.diag);
+      for (int c = 0; c < n; ++c) {
+        const dm::RowRec<W> r = dm::row_rec<W>(rec.data(), t.id[c]);
+        for (int k = 0; k < W; ++k) {
+          jout[size_t(k) * n + c] = c + r.off[k];
+          vout[size_t(k) * n + c] = r.v[k];
+        }
+        dout[c] = r.d;
+      }
+    }
+  });
+  return t.rows;
 }
 int hc_amg_solve(int n, int w, const int* nbr, const double* coef, const double* diag, const double* b, double* xv,
                  double rtol, double atol, int maxit, int nullspace, int mixed, const double cfg[5], int* its,
@@ -184,7 +214,8 @@ int hc_amg_solve(int n, int w, const int* nbr, const double* coef, const double*
     A.diag = diag;
     std::vector<uint32_t> pr;  // the direction pass's compact operator, as the solver attaches it
     std::vector<float> oc;
-    if (mixed && dm::off16_enabled() && dm::ell_pack32(nbr, coef, n, w, pr, oc, A.obase)) {
+    amg.share_rows(A);
+    if (mixed && !A.rid && dm::off16_enabled() && dm::ell_pack32(nbr, coef, n, w, pr, oc, A.obase)) {
       A.opair = pr.data();
       A.ocoef = oc.data();
     }

@@ -1,6 +1,8 @@
 """The multigrid cycle's sparse products and its dense bottom: with no level, some or all of them
 folded into the dense product it is the statement's cycle, on the CPU (host-check build) and as the
-GPU's preconditioner."""
+GPU's preconditioner. The row table of the level-0 passes holds the lists' rows."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -9,8 +11,8 @@ import oracle.amg as om
 from dopamine_amd import cases
 from dopamine_amd.solver import FVSolver
 from helpers import rel_l2, run_case
-from hostcheck import AMG_DEFAULTS, amg_vcycle, lib
-from test_amg import OPERATORS, chain, operator
+from hostcheck import AMG_DEFAULTS, amg_solve, amg_vcycle, lib
+from test_amg import OPERATORS, box_ell, chain, operator
 
 @pytest.fixture(params=[0, 300, 1 << 20])
 def dense(request):
@@ -53,14 +55,76 @@ def test_cells_without_couplings(dense):
     assert np.linalg.norm(z - zo) <= 5e-4 * np.linalg.norm(zo)
 
 
+def row_table(nbr, coef, diag, share):
+    """(distinct rows, neighbours, coefficients, diagonal) as the passes read them; rows 0: no table."""
+    nbr = np.ascontiguousarray(nbr, dtype=np.int32)
+    coef, diag = np.ascontiguousarray(coef, dtype=np.float64), np.ascontiguousarray(diag, dtype=np.float64)
+    w, n = nbr.shape
+    width = ctypes.c_int(0)
+    j, v, d = np.zeros(8 * n, np.int32), np.zeros(8 * n, np.float32), np.zeros(n, np.float32)
+    ptr = lambda a: ctypes.c_void_p(a.ctypes.data)  # noqa: E731
+    rows = lib().hc_row_table(n, w, ptr(nbr), ptr(coef), ptr(diag), share, ctypes.byref(width), ptr(j), ptr(v), ptr(d))
+    W = width.value
+    return rows, j[: W * n].reshape(W, n), v[: W * n].reshape(W, n), d
+
+
+@pytest.mark.parametrize("name,share", [("box", 16), ("channel", 4), ("full_stack", 2), ("tgv_skew", 1), ("tets", 1)])
+def test_row_table_holds_the_lists(name, share):
+    if name == "box":
+        nbr = box_ell(9, 8, 7)
+        coef = np.where(nbr >= 0, 1.0, 0.0)
+        nbr, order = np.sort(nbr, axis=0), np.argsort(nbr, axis=0)  # one slot order for all cells
+        coef = np.take_along_axis(coef, order, 0)
+        diag = coef.sum(axis=0)
+    else:
+        nbr, coef, diag, _ = operator(OPERATORS[name]())
+    rows, j, v, d = row_table(nbr, coef, diag, share)
+    n = nbr.shape[1]
+    assert 0 < rows <= n // share
+    live = nbr >= 0
+    for k in range(len(j)):
+        has = live[k] if k < len(nbr) else np.zeros(n, bool)
+        assert np.array_equal(j[k], np.where(has, nbr[k] if k < len(nbr) else 0, np.arange(n)))
+        assert np.array_equal(v[k], np.where(has, coef[k] if k < len(nbr) else 0.0, 0.0).astype(np.float32))
+    assert np.array_equal(d, diag.astype(np.float32))
+
+
+def test_no_row_table():
+    nbr, coef, diag, _ = operator(OPERATORS["tets"]())
+    assert row_table(nbr, coef, diag, 16)[0] == 0  # jittered: a row per cell
+    nbr, coef, diag, _ = operator(OPERATORS["channel"]())
+    assert row_table(nbr, coef, diag, 0)[0] == 0
+    assert row_table(np.vstack([nbr, nbr]), np.vstack([coef, coef]), diag, 1)[0] == 0  # 12 slots
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("name", ["channel", "full_stack", "tets"])
+def test_row_table_solve_is_the_lists_solve(name, mixed, monkeypatch):
+    """The table holds the lists' values in the lists' slots: the same solve, bit for bit."""
+    nbr, coef, diag, ns = operator(OPERATORS[name]())
+    b = np.random.default_rng(4).standard_normal(diag.size)
+    b -= b.mean()
+    out = []
+    for share, off16 in ((1, "1"), (0, "0")):
+        monkeypatch.setenv("DOPAMINE_ELL_OFF16", off16)
+        lib().hc_amg_row_share(share)
+        try:
+            out.append(amg_solve(nbr, coef, diag, b, 1e-8, nullspace=ns, mixed=mixed))
+        finally:
+            lib().hc_amg_row_share(-1)
+    assert out[0][0] == 0 and out[0][2] == out[1][2] and np.array_equal(out[0][1], out[1][1])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("folded", [0, 300])
-@pytest.mark.parametrize("name", ["tets", "full_stack"])
-def test_gpu_deep_cycles_track_the_oracle(name, folded, precision, monkeypatch):
+@pytest.mark.parametrize("folded,share", [(0, 0), (300, 0), (300, 1)])
+@pytest.mark.parametrize("name", ["tets", "full_stack", "channel"])
+def test_gpu_deep_cycles_track_the_oracle(name, folded, share, precision, monkeypatch):
     """Two steps at p_tol 1e-8 against the oracle's Jacobi CG at 1e-12, as the multigrid tests."""
     case = {"tets": lambda: cases.cavity_tets(6, rcm=True),
-            "full_stack": lambda: cases.full_stack(16, 16, 8, n_obstacles=3, seed=5)}[name]()
+            "full_stack": lambda: cases.full_stack(16, 16, 8, n_obstacles=3, seed=5),
+            "channel": lambda: cases.small_channel(18, 13, 11)}[name]()
+    monkeypatch.setenv("DOPAMINE_AMG_ROW_SHARE", str(share))
     monkeypatch.setenv("DOPAMINE_AMG_COARSE", "64")
     monkeypatch.setenv("DOPAMINE_AMG_DENSE", str(folded))
     mesh = case.make_mesh()
@@ -68,7 +132,7 @@ def test_gpu_deep_cycles_track_the_oracle(name, folded, precision, monkeypatch):
     o = oracle.Solver(mesh, case.params)
     run_case(o, case, mesh, nsteps=2, stats_every=2)
     case.params.p_tol, case.params.precond = 1e-8, "MULTIGRID"
-    print(f"[gpu] multigrid {name}, folded up to {folded}, precision {precision}", flush=True)
+    print(f"[gpu] multigrid {name}, folded up to {folded}, row share {share}, precision {precision}", flush=True)
     g = FVSolver(mesh, case.params, precision=precision)
     run_case(g, case, mesh, nsteps=2, stats_every=2)
     assert g.multigrid_info()["levels"] >= 3 and g.retries == 0
