@@ -360,6 +360,10 @@ struct AmgCfg {
   int dense_max = 2816;
   // Level 0 takes the row table where it has at least this many cells per distinct row (0: never).
   int row_share = 16;
+  // With a row table, level 0 of at least this many cells restricts through Down0 and Gather0
+  // instead of R: 40 + 20 us for 93 us on 7.9 million cells (FP32), 28 + 16 us for 55 us on 4.3
+  // million (FP64); on 0.5 to 0.8 million cells R is as fast or 2% faster over the whole step.
+  int down_cells = 1 << 20;
   int max_levels = 16;
 };
 
@@ -438,15 +442,17 @@ struct AmgMat {
 struct AmgLevelDev {
   int n = 0, w = 0;                              // cells; ELL width (level 0 only)
   const int* nbr = nullptr;                      // level 0: ELL neighbours [slot][cell]
-  const AmgCoef *cs = nullptr, *cr = nullptr;    // level 0: scaled couplings [slot][cell]
+  const AmgCoef* cr = nullptr;                   // level 0: scaled couplings [slot][cell]
   // level 0, when its neighbour offsets fit 16 bits (EllOff16): each slot's coupling and offset
   // in one word (binary16 coupling in the low half, offset - obase[slot] in the high half)
   const uint32_t* hr = nullptr;
   int obase[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   // or, when the operator has a row table (RowTable): the row of each cell and the post-smoothing's
-  // records (offsets, cr, 1 / diag)
+  // records (offsets, cr, 1 / diag); on large levels also the pre-smoothing's (offsets, cs) and the
+  // aggregates' cells, packed rows padded with -1
   const uint16_t* rid = nullptr;
-  const void* rup = nullptr;
+  const void *rup = nullptr, *rdown = nullptr;
+  const int *kptr = nullptr, *kidx = nullptr;
   const float* dinv = nullptr;
   AmgMat<AmgCoef> S;                             // coarse levels: the couplings cs
   AmgMat<float> R, Q;                            // R to the next level; coarse levels: Q = R^T
@@ -699,6 +705,70 @@ struct Restrict0 {
   }
 };
 
+// Level 0 on the way down where it has a row table and many cells (AmgCfg::down_cells): the
+// residual after the pre-smoothing of every cell, r = (1 - w) b + w sum_j cs_j b_j, as a chained
+// pass (10 bytes a cell from memory), then its sum over each aggregate's cells. R, which holds 29
+// bytes a cell, is bound by its own stream there.
+template <class T, int WC>
+struct Down0 {
+  static constexpr bool kPre = true;
+  AmgLevelDev L;
+  const T* b;
+  float* r;
+  CgScalars* sc;
+  int mode, k;
+  float omega;
+  using Scal = cgk::NoScal;
+  struct Pre {
+    float h[WC], bj[WC], bc;
+  };
+  DM_HD cgk::Head head() const { return sc ? cgk::read_head(sc, 0) : cgk::Head{}; }
+  DM_HD bool setup(const Red<1>& t, bool leader, Scal&, const cgk::Head& h) const {
+    return cycle_test(sc, h, mode, k, t.v[0], leader);
+  }
+  DM_HD Pre load(int c) const {
+    Pre o;
+    o.bc = float(b[c]);
+    const RowRec<WC> row = row_rec<WC>(L.rdown, L.rid[c]);
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) {
+      o.h[kk] = row.v[kk];
+      o.bj[kk] = float(b[c + row.off[kk]]);
+    }
+    return o;
+  }
+  DM_HD void apply(int c, const Pre& o, const Scal&, Red<0>&) const {
+    float s = 0.0f;
+#pragma unroll
+    for (int kk = 0; kk < WC; ++kk) s = s + o.h[kk] * o.bj[kk];
+    r[c] = (1.0f - omega) * o.bc + omega * s;
+  }
+};
+struct Gather0 {
+  const int *kptr, *kidx;
+  const float* r;
+  float* bn;
+  const CgScalars* sc;
+  int mode;
+  DM_HD void operator()(int t) const {
+    int lane, st;
+    if (!group_lane<AMG_GU>(t, &lane, &st)) return;
+    if (gated(sc, mode)) return;
+    const int I = t / AMG_GU, q0 = kptr[I], ng = kptr[I + 1] - q0;
+    float s = 0.0f;
+    for (int g = lane; g < ng; g += st) {
+      const AmgI4 i = *reinterpret_cast<const AmgI4*>(kidx + size_t(q0 + g) * AMG_UN);
+      float v[AMG_UN];
+#pragma unroll
+      for (int u = 0; u < AMG_UN; ++u) v[u] = i.v[u] >= 0 ? r[i.v[u]] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < AMG_UN; ++u) s = s + v[u];
+    }
+    s = group_sum<AMG_GU>(s);
+    if (lane == 0) bn[I] = s;
+  }
+};
+
 // A coarse level on the way up: y = w D^-1 ((2 - w) b + w sum_j cs_j b_j) + alpha Q y_next, the
 // pre-smoothing, the coarse correction and the post-smoothing in one.
 struct UpS {
@@ -926,7 +996,20 @@ class AmgPc : public FcgPc, public FcgPc32 {
         L.agg = up(agg);
         L.x = fresh<float>(cur.n);
       }
-      res.push_back(amg_restriction(cur, cfg.omega, na, ptr, idx, scaled));
+      if (L.rdown) {
+        std::vector<int> kptr(size_t(na) + 1, 0), kidx;
+        kidx.reserve(idx.size() + size_t(na) * 2);
+        for (int I = 0; I < na; ++I) {
+          kidx.insert(kidx.end(), idx.begin() + ptr[I], idx.begin() + ptr[I + 1]);
+          kidx.resize((kidx.size() + AMG_UN - 1) / AMG_UN * AMG_UN, -1);
+          kptr[size_t(I) + 1] = int(kidx.size() / AMG_UN);
+        }
+        L.kptr = up(kptr);
+        L.kidx = up(kidx);
+        res.emplace_back();
+      } else {
+        res.push_back(amg_restriction(cur, cfg.omega, na, ptr, idx, scaled));
+      }
       AmgOp next = amg_galerkin(cur, agg, na, ptr, idx);
       levels_.push_back(L);
       ops.push_back(std::move(next));
@@ -957,7 +1040,7 @@ class AmgPc : public FcgPc, public FcgPc32 {
     };
     for (int l = 0; l < bottom_; ++l) {
       AmgLevelDev& L = levels_[size_t(l)];
-      put(res[size_t(l)], levels_[size_t(l) + 1].n, L.R);
+      if (!L.rdown) put(res[size_t(l)], levels_[size_t(l) + 1].n, L.R);
       if (l > 0) put(amg_transpose(res[size_t(l)], L.n), L.n, L.Q);
     }
     levels_[0].yc = levels_[1].y;
@@ -1021,7 +1104,6 @@ class AmgPc : public FcgPc, public FcgPc32 {
         cr[q] = float(cur.coef[q] / cur.diag[c]);
       }
     const std::vector<AmgCoef> hcs = to_coef(cs), hcr = to_coef(cr);
-    L.cs = up(hcs);
     L.cr = up(hcr);
     if (!off16_enabled()) return;
     RowTable t;
@@ -1035,6 +1117,7 @@ class AmgPc : public FcgPc, public FcgPc32 {
         constexpr int W = decltype(wc)::value;
         if constexpr (W > 0) {
           L.rup = up(row_recs<W>(t, t.cr, t.dinv));
+          if (cur.n >= cfg_.down_cells) L.rdown = up(row_recs<W>(t, t.cs, t.dinv));
           rdir_ = up(row_recs<W>(t, t.coef, t.diag));
         }
       });
@@ -1096,9 +1179,20 @@ class AmgPc : public FcgPc, public FcgPc32 {
     const int n1 = levels_[1].n;
     float* b1 = levels_[1].b;
     xx.tbegin(K_MG_DOWN);
-    xx.template pass<1, 0>(n1 * amgk::AMG_GR, amgk::Restrict0<T>{L0.R, r, b1, sc, mode, k}, rr_part, rr_g,
-                           (double*)nullptr);
-    xx.tend(K_MG_DOWN);
+    if (L0.rdown) {
+      with_width(L0.w, [&](auto wc) {
+        constexpr int WC = decltype(wc)::value;
+        if constexpr (WC > 0)
+          xx.template pass<1, 0>(L0.n, amgk::Down0<T, WC>{L0, r, L0.x, sc, mode, k, om}, rr_part, rr_g,
+                                 (double*)nullptr);
+      });
+      xx.tend(K_MG_DOWN);
+      xx.for_each(n1 * amgk::AMG_GU, amgk::Gather0{L0.kptr, L0.kidx, L0.x, b1, sc, mode});
+    } else {
+      xx.template pass<1, 0>(n1 * amgk::AMG_GR, amgk::Restrict0<T>{L0.R, r, b1, sc, mode, k}, rr_part, rr_g,
+                             (double*)nullptr);
+      xx.tend(K_MG_DOWN);
+    }
     for (int l = 1; l < bottom_; ++l) {
       const AmgLevelDev &C = levels_[size_t(l)], &N = levels_[size_t(l) + 1];
       xx.for_each(N.n * amgk::AMG_GR, amgk::RestrictS{C.R, C.b, N.b, sc, mode});

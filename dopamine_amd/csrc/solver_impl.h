@@ -242,7 +242,8 @@ class SolverT {
   // Multigrid set-up: AmgCfg's defaults; DOPAMINE_AMG_THETA / _THETA0 / _ALPHA / _COARSE override
   // the strength thresholds (all levels / the first), the coarse-correction scaling and the
   // densely solved size; _DENSE the size up to which levels are folded into it, _ROW_SHARE the
-  // cells per distinct row from which the row table is used.
+  // cells per distinct row from which the row table is used, _DOWN_CELLS the cells from which it
+  // takes the way down.
   static AmgCfg amg_cfg() {
     AmgCfg c;
     if (const char* e = std::getenv("DOPAMINE_AMG_THETA")) c.theta = std::atof(e);
@@ -253,6 +254,7 @@ class SolverT {
     if (const char* e = std::getenv("DOPAMINE_AMG_COARSE")) c.coarse_max = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("DOPAMINE_AMG_DENSE")) c.dense_max = std::atoi(e);
     if (const char* e = std::getenv("DOPAMINE_AMG_ROW_SHARE")) c.row_share = std::atoi(e);
+    if (const char* e = std::getenv("DOPAMINE_AMG_DOWN_CELLS")) c.down_cells = std::atoi(e);
     return c;
   }
   static double mixed_tau() {

@@ -141,14 +141,17 @@ int hc_ell_off16(int n, int w, const int* nbr, int* base, int16_t* d, int* src) 
 }
 // Size up to which levels are folded into the cycle's dense bottom (AmgCfg::dense_max; negative:
 // the product's).
-static int g_dense_max = -1, g_row_share = -1;
+static int g_dense_max = -1, g_row_share = -1, g_down_cells = -1;
 void hc_amg_dense_max(int m) { g_dense_max = m; }
 // Cells per distinct row from which level 0 takes the row table (AmgCfg::row_share; 0 never,
 // negative the product's).
 void hc_amg_row_share(int m) { g_row_share = m; }
+// Cells from which a level 0 with a row table restricts through it (AmgCfg::down_cells).
+void hc_amg_down_cells(int m) { g_down_cells = m; }
 static void layout(dm::AmgCfg& c) {
   if (g_dense_max >= 0) c.dense_max = g_dense_max;
   if (g_row_share >= 0) c.row_share = g_row_share;
+  if (g_down_cells >= 0) c.down_cells = g_down_cells;
 }
 // The row table of an ELL operator with unit couplings: the number of distinct rows (0: none) and,
 // through the pass's record reader, every cell's neighbours and coefficients (W * n, empty slots

@@ -36,6 +36,24 @@ def test_cycle_matches_the_statement(name, dense):
     assert np.linalg.norm(z - zo) <= 5e-4 * np.linalg.norm(zo)
 
 
+@pytest.mark.parametrize("name", ["tgv_skew", "hydro", "full_stack", "channel"])
+def test_cycle_through_the_row_table(name):
+    """Level 0 restricting through its row table (the form of the large operators)."""
+    nbr, coef, diag, _ = operator(OPERATORS[name]())
+    H = om.Hierarchy(nbr, coef, diag, *AMG_DEFAULTS)
+    r = np.random.default_rng(6).standard_normal(diag.size)
+    lib().hc_amg_row_share(1)
+    lib().hc_amg_down_cells(0)
+    try:
+        z, _, sizes = amg_vcycle(nbr, coef, diag, r)
+    finally:
+        lib().hc_amg_row_share(-1)
+        lib().hc_amg_down_cells(-1)
+    assert sizes == H.sizes
+    zo = H.vcycle(r)
+    assert np.linalg.norm(z - zo) <= 5e-4 * np.linalg.norm(zo)
+
+
 def test_cells_without_couplings(dense):
     """A chain with isolated cells: rows with no couplings and aggregates of one cell."""
     nbr, coef, diag = chain(257, dirichlet=1.0)
@@ -117,14 +135,16 @@ def test_row_table_solve_is_the_lists_solve(name, mixed, monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("folded,share", [(0, 0), (300, 0), (300, 1)])
+@pytest.mark.parametrize("folded,share", [(0, 0), (300, 0), (300, 1), (300, "1 down")])
 @pytest.mark.parametrize("name", ["tets", "full_stack", "channel"])
 def test_gpu_deep_cycles_track_the_oracle(name, folded, share, precision, monkeypatch):
     """Two steps at p_tol 1e-8 against the oracle's Jacobi CG at 1e-12, as the multigrid tests."""
     case = {"tets": lambda: cases.cavity_tets(6, rcm=True),
             "full_stack": lambda: cases.full_stack(16, 16, 8, n_obstacles=3, seed=5),
             "channel": lambda: cases.small_channel(18, 13, 11)}[name]()
-    monkeypatch.setenv("DOPAMINE_AMG_ROW_SHARE", str(share))
+    monkeypatch.setenv("DOPAMINE_AMG_ROW_SHARE", str(share)[0])
+    if share == "1 down":  # restricting through the row table
+        monkeypatch.setenv("DOPAMINE_AMG_DOWN_CELLS", "0")
     monkeypatch.setenv("DOPAMINE_AMG_COARSE", "64")
     monkeypatch.setenv("DOPAMINE_AMG_DENSE", str(folded))
     mesh = case.make_mesh()
