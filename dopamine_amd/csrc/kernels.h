@@ -21,6 +21,10 @@ struct DevMesh {
   const int *nB, *bface, *both, *bidx;            // projection-face list, ELL wB x nc
   const int *nL, *lidx;                           // LS stencil, ELL wL x nc
   const double* lw;                               // LS weights: plane (3k+i) of nc values
+  // or, instead of lw, what the weights are made of (LsRow): the inverse normal matrix of each cell
+  // (6 planes: 00 01 02 11 12 22) and the displacement to each boundary face's pseudo-neighbour or
+  // periodic neighbour; lidx then holds -1 - b and -1 - nb - b for these
+  const double *lsa = nullptr, *lsd = nullptr;
   // faces
   const double *sf, *gc, *area, *nrm, *eps, *wbl, *fctr, *dcf;
   const int *fown, *fnb;                          // face owner / neighbour (-1 on boundary faces)
@@ -251,43 +255,88 @@ DM_INLINE double sgs_nu(int sgs, const double* g, const double* G, double c_v, d
   return 0.0;
 }
 
-// ls_gradient_vector (src/numerics/mod_gradient.f90:425-556), optionally followed by the SGS
-// viscosity of the same cell (sgs: 0 none, 1 Vreman, 2 Smagorinsky, 3 AMD, -1 leave nu_sgs alone).
-struct LsGradVec {
-  DevMesh M;
-  const double *U, *Ub;
-  double *grad, *nu_sgs;
-  int sgs;
-  double c_v, cs, c_amd, dt_stab;
-  DM_HD void operator()(int c) const {
-    const int nc = M.nc;
-    const double u0 = U[3 * size_t(c)], u1 = U[3 * size_t(c) + 1], u2 = U[3 * size_t(c) + 2];
-    double g[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const int cnt = M.nL[c];
-    for (int k = 0; k < cnt; ++k) {
-      const size_t s = size_t(k) * nc + c;
-      const int j = M.lidx[s];
-      const double* un = (j >= 0) ? &U[3 * size_t(j)] : &Ub[3 * size_t(-1 - j)];
-      const double du[3] = {un[0] - u0, un[1] - u1, un[2] - u2};
-      const double w0 = M.lw[(3 * size_t(k)) * nc + c], w1 = M.lw[(3 * size_t(k) + 1) * nc + c],
-                   w2 = M.lw[(3 * size_t(k) + 2) * nc + c];
-      for (int q = 0; q < 3; ++q) {
-        g[3 * q + 0] = g[3 * q + 0] + w0 * du[q];
-        g[3 * q + 1] = g[3 * q + 1] + w1 * du[q];
-        g[3 * q + 2] = g[3 * q + 2] + w2 * du[q];
+// One cell's least-squares stencil: visit(at, w0, w1, w2) gets each neighbour (at >= 0 a cell, else
+// boundary value -1 - at) with its weight, in list order.
+//
+// GEO = 0 reads the weights: 24 bytes per neighbour from memory, 624 of the 830 bytes a hex cell's
+// velocity gradient moves. GEO = 1 forms them: a weight is Ai d / |d|^2 (inverse-distance normal
+// equations), so the loop visits with d / |d|^2, d from the two centroids (gathered through L2 as
+// the velocities are), and finish() applies the cell's Ai (48 bytes) to the sums. What bounds it
+// then is the gathers' latency, so K entries' indices and then their operands travel together, the
+// rest of the last K being the cell itself with weight 0; boundary entries differ from cells in
+// their addresses only.
+template <int GEO>
+struct LsRow {
+  template <int K, class V>
+  DM_HD static void each(const DevMesh& M, int c, V&& visit) {
+    const int nc = M.nc, cnt = M.nL[c];
+    if constexpr (GEO) {
+      const double x0 = M.ctr[3 * size_t(c)], x1 = M.ctr[3 * size_t(c) + 1], x2 = M.ctr[3 * size_t(c) + 2];
+      int jn[K];
+#pragma unroll
+      for (int u = 0; u < K; ++u) jn[u] = u < cnt ? M.lidx[size_t(u) * nc + c] : c;
+      for (int k = 0; k < cnt; k += K) {
+        int at[K];
+        double w[K][3];
+        bool per = false;
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+          const int j = jn[u], e = -1 - j;
+          const double* p = j >= 0 ? &M.ctr[3 * size_t(j)] : &M.lsd[3 * size_t(e < M.nb ? e : e - M.nb)];
+          w[u][0] = p[0] - (j >= 0 ? x0 : 0.0);
+          w[u][1] = p[1] - (j >= 0 ? x1 : 0.0);
+          w[u][2] = p[2] - (j >= 0 ? x2 : 0.0);
+          at[u] = j;
+          per = per || e >= M.nb;
+        }
+        if (per) {
+#pragma unroll
+          for (int u = 0; u < K; ++u)
+            if (-1 - at[u] >= M.nb) at[u] = M.pnb[-1 - at[u] - M.nb];
+        }
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+          const int kn = k + K + u;
+          jn[u] = M.lidx[size_t(kn < cnt ? kn : 0) * nc + c];
+          jn[u] = kn < cnt ? jn[u] : c;
+        }
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+          const double dd = w[u][0] * w[u][0] + w[u][1] * w[u][1] + w[u][2] * w[u][2];
+          const double ww = dd > 0.0 ? 1.0 / dd : 0.0;
+          visit(at[u], ww * w[u][0], ww * w[u][1], ww * w[u][2]);
+        }
+      }
+    } else {
+      for (int k = 0; k < cnt; ++k)
+        visit(M.lidx[size_t(k) * nc + c], M.lw[(3 * size_t(k)) * nc + c], M.lw[(3 * size_t(k) + 1) * nc + c],
+              M.lw[(3 * size_t(k) + 2) * nc + c]);
+    }
+  }
+  // N gradients' sums g[3 q + i] to gradients
+  template <int N>
+  DM_HD static void finish(const DevMesh& M, int c, double* g) {
+    if constexpr (GEO) {
+      const size_t nc = size_t(M.nc);
+      double a[6];
+      for (int i = 0; i < 6; ++i) a[i] = M.lsa[size_t(i) * nc + c];
+      for (int q = 0; q < N; ++q) {
+        const double s0 = g[3 * q], s1 = g[3 * q + 1], s2 = g[3 * q + 2];
+        g[3 * q] = a[0] * s0 + a[1] * s1 + a[2] * s2;
+        g[3 * q + 1] = a[1] * s0 + a[3] * s1 + a[4] * s2;
+        g[3 * q + 2] = a[2] * s0 + a[4] * s1 + a[5] * s2;
       }
     }
-    for (int q = 0; q < 9; ++q) grad[9 * size_t(c) + q] = g[q];
-    if (sgs >= 0) nu_sgs[c] = sgs_nu(sgs, g, &M.Gf[9 * size_t(c)], c_v, cs, c_amd, M.vol[c], dt_stab);
   }
 };
 
-// compute_all_gradients with least squares (src/solver/mod_fv_solver.f90:1003-1077): the velocity
-// gradient (+ SGS viscosity, as LsGradVec) and NSF scalar gradients (temperature, passive scalars,
-// as LsGradSca) in one pass over the stencil, so its indices and weights are read once. Each field
-// accumulates in the same order as its own kernel: the results are those kernels' bit for bit.
+// ls_gradient_vector (src/numerics/mod_gradient.f90:425-556), optionally followed by the SGS
+// viscosity of the same cell (sgs: 0 none, 1 Vreman, 2 Smagorinsky, 3 AMD, -1 leave nu_sgs alone),
+// and NSF scalar gradients (temperature, passive scalars, as LsGradSca; compute_all_gradients,
+// src/solver/mod_fv_solver.f90:1003-1077) in one pass over the stencil. Each field accumulates in
+// the same order as its own kernel: the results are those kernels' bit for bit.
 constexpr int LS_MAX_SCALARS = 5;
-template <int NSF>
+template <int NSF, int GEO>
 struct LsGradAll {
   // the velocity-only form fits five wavefronts per SIMD without spilling (2% faster measured);
   // the forms with scalars would spill
@@ -301,23 +350,17 @@ struct LsGradAll {
   const double* sb[LS_MAX_SCALARS];
   double* sg[LS_MAX_SCALARS];
   DM_HD void operator()(int c) const {
-    const int nc = M.nc;
     const double u0 = U[3 * size_t(c)], u1 = U[3 * size_t(c) + 1], u2 = U[3 * size_t(c) + 2];
     double g[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double pc[NSF > 0 ? NSF : 1], gs[NSF > 0 ? NSF : 1][3];
+    double pc[NSF > 0 ? NSF : 1], gs[NSF > 0 ? 3 * NSF : 1];
 #pragma unroll
     for (int i = 0; i < NSF; ++i) {
       pc[i] = sa[i][c];
-      gs[i][0] = gs[i][1] = gs[i][2] = 0.0;
+      gs[3 * i] = gs[3 * i + 1] = gs[3 * i + 2] = 0.0;
     }
-    const int cnt = M.nL[c];
-    for (int k = 0; k < cnt; ++k) {
-      const size_t s = size_t(k) * nc + c;
-      const int j = M.lidx[s];
+    LsRow<GEO>::template each<NSF == 0 ? 3 : 2>(M, c, [&](int j, double w0, double w1, double w2) {
       const double* un = (j >= 0) ? &U[3 * size_t(j)] : &Ub[3 * size_t(-1 - j)];
       const double du[3] = {un[0] - u0, un[1] - u1, un[2] - u2};
-      const double w0 = M.lw[(3 * size_t(k)) * nc + c], w1 = M.lw[(3 * size_t(k) + 1) * nc + c],
-                   w2 = M.lw[(3 * size_t(k) + 2) * nc + c];
       for (int q = 0; q < 3; ++q) {
         g[3 * q + 0] = g[3 * q + 0] + w0 * du[q];
         g[3 * q + 1] = g[3 * q + 1] + w1 * du[q];
@@ -326,21 +369,26 @@ struct LsGradAll {
 #pragma unroll
       for (int i = 0; i < NSF; ++i) {
         const double d = ((j >= 0) ? sa[i][j] : sb[i][-1 - j]) - pc[i];
-        gs[i][0] = gs[i][0] + w0 * d;
-        gs[i][1] = gs[i][1] + w1 * d;
-        gs[i][2] = gs[i][2] + w2 * d;
+        gs[3 * i] = gs[3 * i] + w0 * d;
+        gs[3 * i + 1] = gs[3 * i + 1] + w1 * d;
+        gs[3 * i + 2] = gs[3 * i + 2] + w2 * d;
       }
-    }
+    });
+    LsRow<GEO>::template finish<3>(M, c, g);
     for (int q = 0; q < 9; ++q) grad[9 * size_t(c) + q] = g[q];
     if (sgs >= 0) nu_sgs[c] = sgs_nu(sgs, g, &M.Gf[9 * size_t(c)], c_v, cs, c_amd, M.vol[c], dt_stab);
+    if constexpr (NSF > 0) {
+      LsRow<GEO>::template finish<NSF>(M, c, gs);
 #pragma unroll
-    for (int i = 0; i < NSF; ++i)
-      for (int q = 0; q < 3; ++q) sg[i][3 * size_t(c) + q] = gs[i][q];
+      for (int i = 0; i < NSF; ++i)
+        for (int q = 0; q < 3; ++q) sg[i][3 * size_t(c) + q] = gs[3 * i + q];
+    }
   }
 };
 
 // ls_gradient_scalar (src/numerics/mod_gradient.f90:307-422) of phi = a (+ a2) with boundary
 // values pb (+ pb2).
+template <int GEO>
 struct LsGradSca {
   DevMesh M;
   const double *a, *a2, *pb, *pb2;
@@ -348,27 +396,23 @@ struct LsGradSca {
   DM_HD double cv(int c) const { return a2 ? a[c] + a2[c] : a[c]; }
   DM_HD double bv(int b) const { return pb2 ? pb[b] + pb2[b] : pb[b]; }
   DM_HD void operator()(int c) const {
-    const int nc = M.nc;
     const double pc = cv(c);
-    double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    const int cnt = M.nL[c];
-    for (int k = 0; k < cnt; ++k) {
-      const size_t s = size_t(k) * nc + c;
-      const int j = M.lidx[s];
+    double s[3] = {0.0, 0.0, 0.0};
+    LsRow<GEO>::template each<4>(M, c, [&](int j, double w0, double w1, double w2) {
       const double d = ((j >= 0) ? cv(j) : bv(-1 - j)) - pc;
-      g0 = g0 + M.lw[(3 * size_t(k)) * nc + c] * d;
-      g1 = g1 + M.lw[(3 * size_t(k) + 1) * nc + c] * d;
-      g2 = g2 + M.lw[(3 * size_t(k) + 2) * nc + c] * d;
-    }
-    g[3 * size_t(c)] = g0;
-    g[3 * size_t(c) + 1] = g1;
-    g[3 * size_t(c) + 2] = g2;
+      s[0] = s[0] + w0 * d;
+      s[1] = s[1] + w1 * d;
+      s[2] = s[2] + w2 * d;
+    });
+    LsRow<GEO>::template finish<1>(M, c, s);
+    for (int i = 0; i < 3; ++i) g[3 * size_t(c) + i] = s[i];
   }
 };
 
 // LsGradSca on a list of cells only.
+template <int GEO>
 struct LsGradScaAt {
-  LsGradSca g;
+  LsGradSca<GEO> g;
   const int* cells;
   DM_HD void operator()(int i) const { g(cells[i]); }
 };

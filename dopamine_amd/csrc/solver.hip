@@ -442,8 +442,12 @@ int dopamine_op_ls_gradient_vector(void* h, const double* U, const double* U_bnd
     const Sizes z = sizes(s);
     OpBufs b(s->x);
     double* g = b.zeros(9 * z.nc);
-    s->x.for_each(s->nc, dm::LsGradVec{s->M, b.in(U, 3 * z.nc), b.in(U_bnd, 3 * z.nb), g, nullptr, -1, 0.0, 0.0, 0.0,
-                                       0.0});
+    const double* u = b.in(U, 3 * z.nc);
+    const double* ub = b.in(U_bnd, 3 * z.nb);
+    s->ls_dispatch([&](auto geo) {
+      s->x.for_each(s->nc, dm::LsGradAll<0, decltype(geo)::value>{s->M, u, ub, g, nullptr, -1, 0.0, 0.0, 0.0, 0.0, {}, {},
+                                                                  {}});
+    });
     b.out(grad_U, g, 9 * z.nc);
     return 0;
   });
@@ -455,7 +459,11 @@ int dopamine_op_ls_gradient_scalar(void* h, const double* phi, const double* phi
     const Sizes z = sizes(s);
     OpBufs b(s->x);
     double* g = b.zeros(3 * z.nc);
-    s->x.for_each(s->nc, dm::LsGradSca{s->M, b.in(phi, z.nc), nullptr, b.in(phi_bnd, z.nb), nullptr, g});
+    const double* p = b.in(phi, z.nc);
+    const double* pb = b.in(phi_bnd, z.nb);
+    s->ls_dispatch([&](auto geo) {
+      s->x.for_each(s->nc, dm::LsGradSca<decltype(geo)::value>{s->M, p, nullptr, pb, nullptr, g});
+    });
     b.out(grad, g, 3 * z.nc);
     return 0;
   });

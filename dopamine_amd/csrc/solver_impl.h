@@ -29,6 +29,9 @@
 
 namespace dm {
 
+// nearly singular least-squares normal matrices (src/mesh/mod_mesh.f90:513-754), as the mesh set-up
+constexpr double LS_DET_TOL = 1.0e-12, LS_REG_FRAC = 1.0e-6;
+
 struct SolverScalars {
   double divmax, ub1, ub2, atol, pmean, shift, cfl, dif;
   double st[12];
@@ -644,7 +647,17 @@ class SolverT {
     M.ctr = up(vec_d(d.cell_centroid, 3 * size_t(nc)));
     M.nA = up(nA); M.aface = up(aface); M.aoth = up(aoth);
     M.nB = up(nB); M.bface = up(bface); M.both = up(both); M.bidx = up(bidx);
-    M.nL = up(nL); M.lidx = up(lidx); M.lw = up(lw);
+    M.nL = up(nL);
+    {
+      std::vector<double> lsa, lsd;
+      if (ls_geometry(d, pnb, wL, lidx, lsa, lsd)) {
+        M.lsa = up(lsa);
+        M.lsd = up(lsd);
+      } else {
+        M.lw = up(lw);
+      }
+    }
+    M.lidx = up(lidx);
     M.sf = up(vec_d(d.face_sf, 3 * size_t(nf)));
     M.gc = up(vec_d(d.face_gc, nf));
     M.area = up(vec_d(d.face_area, nf));
@@ -949,6 +962,99 @@ class SolverT {
     }
   }
 
+  // Whether the next cell's k-th neighbour is the next cell of this one's for most k, as on meshes
+  // numbered along rows: the gather of the centroids is then a few lines per wavefront and costs less
+  // than the weights (LsRow). Measured, formed / stored: velocity 110 / 157 us on 786,432 hex cells,
+  // 70 / 99 us (with the temperature 72 / 105, one scalar 48 / 77) on 524,288, 18 / 24 us on 98,304,
+  // with three scalars 185 / 195 us on 509,486 (registers allow two entries at a time); on tets,
+  // whose lanes gather from as many lines, the velocity 49 / 39 us on 131,712 cells and 457 / 428 us
+  // on 998,250 (renumbered to a small bandwidth), so these keep the weights.
+  bool consecutive_neighbours(int wL, const std::vector<int>& lidx) const {
+    int64_t next = 0, all = 0;
+    for (int k = 0; k < wL; ++k)
+      for (int c = 0; c + 1 < nc; ++c) {
+        const int a = lidx[size_t(k) * nc + c], b = lidx[size_t(k) * nc + c + 1];
+        all += a >= 0;
+        next += a >= 0 && b == a + 1;
+      }
+    return 2 * next > all;
+  }
+  // The least-squares weights in terms of the geometry (LsRow<1>): entry k < faces of the cell of a
+  // stencil row is the neighbour through the cell's k-th face (a periodic partner at the pair's
+  // distance along the normal, or the boundary face's centre), the others are cells at their
+  // centroids; w = Ai d / |d|^2 with Ai the inverse of sum d d^T / |d|^2, regularised where it is
+  // nearly singular (src/mesh/mod_mesh.f90:513-754). Fills Ai and the boundary displacements and
+  // renumbers lidx; false (nothing changed) unless every weight of the mesh is reproduced to 1e-12
+  // of its row's largest, so weights from elsewhere are taken as they are.
+  bool ls_geometry(const dopamine_mesh_desc& d, const std::vector<int>& pnb, int wL, std::vector<int>& lidx,
+                   std::vector<double>& lsa, std::vector<double>& lsd) const {
+    const char* e = std::getenv("DOPAMINE_LS_GEOMETRY");  // 0, 1: whatever the numbering
+    if (e ? e[0] == '0' : !consecutive_neighbours(wL, lidx)) return false;
+    std::vector<int> enc(lidx);
+    lsa.assign(6 * size_t(nc), 0.0);
+    lsd.assign(3 * size_t(std::max(1, nb)), 0.0);
+    std::vector<double> dv(3 * size_t(std::max(1, wL)));
+    for (int c = 0; c < nc; ++c) {
+      const int off = d.ls_offset[c], cnt = d.ls_offset[c + 1] - off, fo = d.cell_face_offset[c],
+                nfc = d.cell_face_offset[c + 1] - fo;
+      double a[6] = {0, 0, 0, 0, 0, 0};  // 00 01 02 11 12 22
+      for (int k = 0; k < cnt; ++k) {
+        const int cell = d.ls_cell[off + k], f = k < nfc ? d.cell_faces[fo + k] : -1, b = f - nint;
+        double* v = &dv[3 * size_t(k)];
+        const bool per = f >= nint && cell >= 0 && pnb[b] == cell;
+        if (per) {
+          const double dn = d.periodic_pair_dcf[b] > 0.0 ? d.periodic_pair_dcf[b] : d.face_dcf[f];
+          for (int i = 0; i < 3; ++i) v[i] = (d.face_dcf[f] + dn) * d.face_normal[3 * size_t(f) + i];
+        } else if (cell >= 0) {
+          for (int i = 0; i < 3; ++i)
+            v[i] = d.cell_centroid[3 * size_t(cell) + i] - d.cell_centroid[3 * size_t(c) + i];
+        } else {
+          if (f < nint || d.ls_face[off + k] != f) return false;
+          for (int i = 0; i < 3; ++i) v[i] = d.face_centre[3 * size_t(f) + i] - d.cell_centroid[3 * size_t(c) + i];
+        }
+        if (per || cell < 0) {
+          enc[size_t(k) * nc + c] = per ? -1 - nb - b : -1 - b;
+          for (int i = 0; i < 3; ++i) lsd[3 * size_t(b) + i] = v[i];
+        }
+        const double dd = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+        if (!(dd > 0.0) || !std::isfinite(dd)) return false;
+        const double ww = 1.0 / dd;
+        a[0] += ww * v[0] * v[0]; a[1] += ww * v[0] * v[1]; a[2] += ww * v[0] * v[2];
+        a[3] += ww * v[1] * v[1]; a[4] += ww * v[1] * v[2]; a[5] += ww * v[2] * v[2];
+      }
+      const double scale = (a[0] + a[3] + a[5]) / 3.0;
+      double ai[6];
+      const auto invert = [&] {
+        const double c00 = a[3] * a[5] - a[4] * a[4], c01 = a[2] * a[4] - a[1] * a[5], c02 = a[1] * a[4] - a[2] * a[3];
+        const double det = a[0] * c00 + a[1] * c01 + a[2] * c02;
+        ai[0] = c00 / det; ai[1] = c01 / det; ai[2] = c02 / det;
+        ai[3] = (a[0] * a[5] - a[2] * a[2]) / det; ai[4] = (a[1] * a[2] - a[0] * a[4]) / det;
+        ai[5] = (a[0] * a[3] - a[1] * a[1]) / det;
+        return det;
+      };
+      const double det = invert();
+      if (scale <= 0.0 || std::fabs(det) < LS_DET_TOL * scale * scale * scale) {
+        a[0] += LS_REG_FRAC * std::max(scale, SMALL);
+        a[3] += LS_REG_FRAC * std::max(scale, SMALL);
+        a[5] += LS_REG_FRAC * std::max(scale, SMALL);
+        invert();
+      }
+      double wmax = 0.0;
+      for (int k = 0; k < 3 * cnt; ++k) wmax = std::max(wmax, std::fabs(d.ls_weight[3 * size_t(off) + k]));
+      for (int k = 0; k < cnt; ++k) {
+        const double* v = &dv[3 * size_t(k)];
+        const double* w = &d.ls_weight[3 * size_t(off + k)];
+        const double ww = 1.0 / (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+        const double e0 = ww * (ai[0] * v[0] + ai[1] * v[1] + ai[2] * v[2]) - w[0],
+                     e1 = ww * (ai[1] * v[0] + ai[3] * v[1] + ai[4] * v[2]) - w[1],
+                     e2 = ww * (ai[2] * v[0] + ai[4] * v[1] + ai[5] * v[2]) - w[2];
+        if (!(std::fabs(e0) + std::fabs(e1) + std::fabs(e2) <= 1.0e-12 * wmax)) return false;
+      }
+      for (int i = 0; i < 6; ++i) lsa[size_t(i) * nc + c] = ai[i];
+    }
+    lidx.swap(enc);
+    return true;
+  }
   // ---------------------------------------------------------------- boundary passes
 
   void bc_velocity(int filter, const double* gU) { x.for_each(nb, BcVelocity{M, U, gU, U_bnd, filter, out_ready}); }
@@ -1180,6 +1286,14 @@ class SolverT {
     x.for_each(nc, DynNu{M, dyn_lmh, grad, nu_sgs, dt_stab});
   }
 
+  // Calls fn with the form of the mesh's least-squares rows (LsRow).
+  template <class Fn>
+  void ls_dispatch(Fn&& fn) {
+    if (M.lsa)
+      fn(std::integral_constant<int, 1>{});
+    else
+      fn(std::integral_constant<int, 0>{});
+  }
   // bc_only (least squares, no SGS): the velocity gradient everywhere and the temperature gradient
   // only where a boundary value reads it before the next full call; the mid-stage call of the
   // first two stages, whose scalar gradients nothing else reads before the next stage recomputes
@@ -1189,9 +1303,15 @@ class SolverT {
     const int sgs = (with_sgs && !dyn) ? prm.sgs : -1;
     if (prm.gradient == 0 && bc_only && !with_sgs) {
       x.tbegin(K_LS_GRAD);
-      x.for_each(nc, LsGradAll<0>{M, U, U_bnd, grad, nu_sgs, -1, 0.0, 0.0, 0.0, 0.0, {}, {}, {}});
+      ls_dispatch([&](auto geo) {
+        x.for_each(nc, LsGradAll<0, decltype(geo)::value>{M, U, U_bnd, grad, nu_sgs, -1, 0.0, 0.0, 0.0, 0.0, {}, {}, {}});
+      });
       x.tend(K_LS_GRAD);
-      if (bous && n_tbc) x.for_each(n_tbc, LsGradScaAt{LsGradSca{M, T, nullptr, T_bnd, nullptr, gT}, tbc_cell});
+      if (bous && n_tbc)
+        ls_dispatch([&](auto geo) {
+          constexpr int GEO = decltype(geo)::value;
+          x.for_each(n_tbc, LsGradScaAt<GEO>{LsGradSca<GEO>{M, T, nullptr, T_bnd, nullptr, gT}, tbc_cell});
+        });
       return;
     }
     if (prm.gradient == 0) {  // least squares: every field in one pass (LsGradAll)
@@ -1211,14 +1331,16 @@ class SolverT {
       }
       x.tbegin(K_LS_GRAD);
       const auto run = [&](auto n) {
-        constexpr int N = decltype(n)::value;
-        LsGradAll<N> f{M, U, U_bnd, grad, nu_sgs, sgs, prm.c_vreman, prm.cs_smag, prm.c_amd, sgs_dt, {}, {}, {}};
-        for (int i = 0; i < LS_MAX_SCALARS; ++i) {
-          f.sa[i] = sa[i];
-          f.sb[i] = sb[i];
-          f.sg[i] = sg[i];
-        }
-        x.for_each(nc, f);
+        ls_dispatch([&](auto geo) {
+          LsGradAll<decltype(n)::value, decltype(geo)::value> f{M,          U,          U_bnd,     grad,   nu_sgs, sgs,
+                                                                prm.c_vreman, prm.cs_smag, prm.c_amd, sgs_dt, {},     {}, {}};
+          for (int i = 0; i < LS_MAX_SCALARS; ++i) {
+            f.sa[i] = sa[i];
+            f.sb[i] = sb[i];
+            f.sg[i] = sg[i];
+          }
+          x.for_each(nc, f);
+        });
       };
       switch (nsf) {
         case 0: run(std::integral_constant<int, 0>{}); break;
@@ -1235,49 +1357,35 @@ class SolverT {
       return;
     }
     if (bous) {  // compute_all_gradients: the temperature gradient alongside the velocity's
-      if (prm.gradient == 0) {
-        x.for_each(nc, LsGradSca{M, T, nullptr, T_bnd, nullptr, gT});
-      } else {
-        x.for_each(nc, GgGradSca{M, T, nullptr, T_bnd, nullptr, nullptr, gT});
-        for (int it = 2; it <= prm.gg_iterations; ++it) {
-          x.copy(gT_prev, gT, 3 * size_t(nc));
-          x.for_each(nc, GgGradSca{M, T, nullptr, T_bnd, nullptr, gT_prev, gT});
-        }
-      }
-    }
-    for (int k = 0; k < ns; ++k) {  // the scalars' gradients (LS, or GG with its sweeps)
-      if (prm.gradient == 0) {
-        x.for_each(nc, LsGradSca{M, Cs[k], nullptr, Cb[k], nullptr, gC[k]});
-      } else {
-        x.for_each(nc, GgGradSca{M, Cs[k], nullptr, Cb[k], nullptr, nullptr, gC[k]});
-        for (int it = 2; it <= prm.gg_iterations; ++it) {
-          x.copy(gCprev, gC[k], 3 * size_t(nc));
-          x.for_each(nc, GgGradSca{M, Cs[k], nullptr, Cb[k], nullptr, gCprev, gC[k]});
-        }
-      }
-    }
-    if (prm.gradient == 0) {
-      x.tbegin(K_LS_GRAD);
-      x.for_each(nc, LsGradVec{M, U, U_bnd, grad, nu_sgs, sgs, prm.c_vreman, prm.cs_smag, prm.c_amd, sgs_dt});
-      x.tend(K_LS_GRAD);
-    } else {
-      x.for_each(nc, GgGradVec{M, U, U_bnd, nullptr, grad});
+      x.for_each(nc, GgGradSca{M, T, nullptr, T_bnd, nullptr, nullptr, gT});
       for (int it = 2; it <= prm.gg_iterations; ++it) {
-        x.copy(gprev, grad, 9 * size_t(nc));
-        x.for_each(nc, GgGradVec{M, U, U_bnd, gprev, grad});
+        x.copy(gT_prev, gT, 3 * size_t(nc));
+        x.for_each(nc, GgGradSca{M, T, nullptr, T_bnd, nullptr, gT_prev, gT});
       }
-      if (dyn)
-        dynamic_sgs(sgs_dt);
-      else if (with_sgs)
-        x.for_each(nc, SgsCell{M, grad, nu_sgs, prm.sgs, prm.c_vreman, prm.cs_smag, prm.c_amd, sgs_dt});
     }
+    for (int k = 0; k < ns; ++k) {  // the scalars' gradients
+      x.for_each(nc, GgGradSca{M, Cs[k], nullptr, Cb[k], nullptr, nullptr, gC[k]});
+      for (int it = 2; it <= prm.gg_iterations; ++it) {
+        x.copy(gCprev, gC[k], 3 * size_t(nc));
+        x.for_each(nc, GgGradSca{M, Cs[k], nullptr, Cb[k], nullptr, gCprev, gC[k]});
+      }
+    }
+    x.for_each(nc, GgGradVec{M, U, U_bnd, nullptr, grad});
+    for (int it = 2; it <= prm.gg_iterations; ++it) {
+      x.copy(gprev, grad, 9 * size_t(nc));
+      x.for_each(nc, GgGradVec{M, U, U_bnd, gprev, grad});
+    }
+    if (dyn)
+      dynamic_sgs(sgs_dt);
+    else if (with_sgs)
+      x.for_each(nc, SgsCell{M, grad, nu_sgs, prm.sgs, prm.c_vreman, prm.cs_smag, prm.c_amd, sgs_dt});
     if (with_sgs && prm.sgs == 3 && prm.amd_wall_gradient && n_amdw > 0)
       x.for_each(n_amdw, AmdWall{M, amdw_cell, amdw_off, amdw_face, U, grad, nu_sgs, prm.nu, prm.c_amd, sgs_dt});
   }
   // gradient_of_scalar of a (+ a2) with boundary values pb (+ pb2) into gp
   void scalar_gradient(const double* a, const double* a2, const double* pb, const double* pb2) {
     if (prm.gradient == 0) {
-      x.for_each(nc, LsGradSca{M, a, a2, pb, pb2, gp});
+      ls_dispatch([&](auto geo) { x.for_each(nc, LsGradSca<decltype(geo)::value>{M, a, a2, pb, pb2, gp}); });
     } else {
       x.for_each(nc, GgGradSca{M, a, a2, pb, pb2, nullptr, gp});
       for (int it = 2; it <= prm.gg_iterations; ++it) {

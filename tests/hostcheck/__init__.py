@@ -32,6 +32,7 @@ def lib():
         L.hc_solver_stats.argtypes = [ctypes.c_void_p, _d * 8]
         L.hc_solver_time.restype = _d
         L.hc_solver_time.argtypes = [ctypes.c_void_p]
+        L.hc_ls_geometry.argtypes = [ctypes.c_void_p]
         L.hc_solver_counters.argtypes = [ctypes.c_void_p, _i64 * 4]
         L.hc_solver_nonortho_info.argtypes = [ctypes.c_void_p, ctypes.c_int32 * 3]
         L.hc_solver_proj_counters.argtypes = [ctypes.c_void_p, _i64 * 2]
