@@ -219,6 +219,7 @@ class SolverT {
   double *phiC = nullptr, *gCprev = nullptr;
   double* phiCk[4] = {};  // each scalar's face values, for the fused transport of T and the scalars
   double* faceT = nullptr;  // the fused transport's interior-face fluxes, 2 per field and face
+  double* cv_v = nullptr;     // the velocity correction's slots
   TvdCtx* tvd_ctx = nullptr;  // the fused transport's TVD face contexts (both flux signs)
   int* s_mode = nullptr;
   double *s_val = nullptr, *s_flux = nullptr, *s_om = nullptr, *s_ph = nullptr;
@@ -632,6 +633,17 @@ class SolverT {
         if (bbc[b] != BC_PERIODIC) addnn(bown[b], d.face_area[nint + b], &d.face_normal[3 * size_t(nint + b)]);
       for (int c = 0; c < nc; ++c) invert_sym3(&T[9 * size_t(c)], &Tinv[9 * size_t(c)]);
     }
+    // ---- the velocity correction's slots (CorrectVelocity)
+    std::vector<double> cvv(3 * size_t(std::max(1, wB)) * nc, 0.0);
+    for (int c = 0; c < nc; ++c)
+      for (int k = 0; k < nB[c]; ++k) {
+        const size_t q = size_t(k) * nc + c;
+        const double* n = &d.face_normal[3 * size_t(bface[q] >> 1)];
+        const double* t = &Tinv[9 * size_t(c)];
+        const double w = bidx[q] < 0 ? 1.0 : (bface[q] & 1) ? -pcoef[bidx[q]] : pcoef[bidx[q]];
+        for (int i = 0; i < 3; ++i)
+          cvv[size_t(3 * k + i) * nc + c] = w * (t[3 * i] * n[0] + t[3 * i + 1] * n[1] + t[3 * i + 2] * n[2]);
+      }
     // ---- Vreman filter tensor (build_filter_tensor + smooth_filter_tensor)
     std::vector<double> Gf(9 * size_t(nc), 0.0);
     if (p.sgs != 0) build_filter_tensor(d, Gf);
@@ -690,6 +702,7 @@ class SolverT {
     M.pown = up(pown.empty() ? std::vector<int>(1, -1) : pown);
     M.pnbr = up(pnbr.empty() ? std::vector<int>(1, -1) : pnbr);
     M.pfm = up(pfm.empty() ? std::vector<int>(1, 0) : pfm);
+    cv_v = up(cvv);
     M.Tinv = up(Tinv); M.Gf = up(Gf);
     M.patchU = up(patchU_h);
     patchP = up(patchP_h);
@@ -1425,9 +1438,11 @@ class SolverT {
     const int do_cross = (with_cross && !skip_nonortho) ? 1 : 0;
     double fb[3];
     body_force_now(fb);
-    x.for_each(nc, CorrectVelocity{M, P, gp, outlet_pb, U, gpc_out, dt, fb[0], fb[1], fb[2],
-                                   do_cross, ptot ? 1 : 0, bous ? T : nullptr, prm.beta, prm.T_ref, prm.g[0],
-                                   prm.g[1], prm.g[2]});
+    if (do_cross)
+      x.for_each(nc, CorrectVelocityCross{M, P, gp, outlet_pb, U, gpc_out, dt, ptot ? 1 : 0});
+    else
+      x.for_each(nc, CorrectVelocity{M, P, outlet_pb, cv_v, U, gpc_out, dt, fb[0], fb[1], fb[2], ptot ? 1 : 0,
+                                     bous ? T : nullptr, prm.beta, prm.T_ref, prm.g[0], prm.g[1], prm.g[2]});
   }
 
   int pressure_solve(bool ptot, const double* atol_dev, double atol) {
